@@ -278,6 +278,93 @@ __global__ void __launch_bounds__(BLOCK) k_binop_vec(int32_t *result, const int3
     }
 }
 
+// ------------------------------------------------------- tiles of a wave
+
+// Tiles of WT_ROWS rows per wave: chunk j of a lane holds the rows
+// t0 + 256 j + 4 lane .. + 3, so that flags (4 bytes) and columns (16 bytes)
+// load coalesced; bit 4 j + k of a lane's 32-bit row mask is row k of its
+// chunk j.
+constexpr int WT_CHUNKS = 8;
+constexpr int64_t WT_ROWS = 256 * WT_CHUNKS;
+
+__device__ __forceinline__ int64_t wt_row(int64_t t0, int lane, int j) { return t0 + 256 * j + 4 * lane; }
+// offset in its tile of the row of mask bit b
+__device__ __forceinline__ uint32_t wt_offset(int lane, uint32_t b) { return (b >> 2) * 256u + 4u * lane + (b & 3u); }
+
+// Flags of a tile (rows at or past n: 0).  VEC: flags 4-byte aligned.
+template <bool VEC>
+__device__ __forceinline__ void wt_flags(const uint8_t *flags, int64_t n, int64_t t0, int lane, uint32_t (&f)[WT_CHUNKS])
+{
+    if (VEC && t0 + WT_ROWS <= n) {
+#pragma unroll
+        for (int j = 0; j < WT_CHUNKS; j++) f[j] = *reinterpret_cast<const uint32_t *>(flags + wt_row(t0, lane, j));
+        return;
+    }
+#pragma unroll
+    for (int j = 0; j < WT_CHUNKS; j++) {
+        const int64_t r = wt_row(t0, lane, j);
+        f[j] = 0;
+#pragma unroll
+        for (int k = 0; k < 4; k++)
+            if (r + k < n) f[j] |= (uint32_t)flags[r + k] << (8 * k);
+    }
+}
+
+// Bit k: whether byte k of x is nonzero (the flag bits 0, 8, 16, 24 of
+// nz_bytes meet in bits 24..27 of the product, with no carry into them).
+__device__ __forceinline__ uint32_t nz_mask(uint32_t x) { return (nz_bytes(x) * 0x01020408u) >> 24; }
+
+// The flags 0 / 1 of the low four bits of m, one per byte
+__device__ __forceinline__ uint32_t flag_bytes(uint32_t m) { return ((m & 15u) * 0x00204081u) & 0x01010101u; }
+
+__device__ __forceinline__ uint32_t wt_mask(const uint32_t (&f)[WT_CHUNKS])
+{
+    uint32_t m = 0;
+#pragma unroll
+    for (int j = 0; j < WT_CHUNKS; j++) m |= nz_mask(f[j]) << (4 * j);
+    return m;
+}
+
+// LDS written by some lanes of a wave and read by others
+__device__ __forceinline__ void wave_sync()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// Exclusive prefix of v over the lanes of the wave, and the total.
+__device__ __forceinline__ uint32_t wave_prefix(uint32_t v, int lane, uint32_t &total)
+{
+    uint32_t x = v;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const uint32_t y = __shfl_up(x, off, 64);
+        if (lane >= off) x += y;
+    }
+    total = __builtin_amdgcn_readlane(x, 63);
+    return x - v;
+}
+
+// Block-wide min and max (BLOCK threads), valid in thread 0
+__device__ __forceinline__ void block_minmax(int32_t &lo, int32_t &hi)
+{
+    for (int off = 32; off > 0; off >>= 1) {
+        lo = min(lo, __shfl_xor(lo, off, 64));
+        hi = max(hi, __shfl_xor(hi, off, 64));
+    }
+    __shared__ int32_t wlo[BLOCK / 64], whi[BLOCK / 64];
+    if ((threadIdx.x & 63) == 0) {
+        wlo[threadIdx.x >> 6] = lo;
+        whi[threadIdx.x >> 6] = hi;
+    }
+    __syncthreads();
+    for (int w = 0; w < BLOCK / 64; w++) {
+        lo = min(lo, wlo[w]);
+        hi = max(hi, whi[w]);
+    }
+}
+
 // ------------------------------------------------------------------ join
 
 __global__ void __launch_bounds__(BLOCK) k_build_keys(const int32_t *keys, const uint8_t *flags,
@@ -455,60 +542,252 @@ __global__ void __launch_bounds__(BLOCK) k_probe_full(const int32_t *__restrict_
     }
 }
 
-__global__ void k_pairs_range_init(int32_t *info)
-{
-    info[0] = INT32_MAX;
-    info[1] = INT32_MIN;
-    info[2] = 0;
-}
+// Each block's min and max of the values of the slots whose flag is 1, to
+// partials[2 b], [2 b + 1] (no slot set: INT32_MAX, INT32_MIN)
+constexpr unsigned PAIRS_RANGE_BLOCKS = BLOCK; // one partial per thread of the reader
 
-// min and max of the values of the slots whose flag is 1
-__global__ void __launch_bounds__(BLOCK) k_pairs_range(const int2 *pairs, int64_t len, int32_t *info)
+__global__ void __launch_bounds__(BLOCK) k_pairs_range(const int2 *__restrict__ pairs, int64_t len, int32_t *partials)
 {
     int32_t lo = INT32_MAX, hi = INT32_MIN;
-    for (int64_t h = (int64_t)blockIdx.x * BLOCK + threadIdx.x; h < len; h += (int64_t)gridDim.x * BLOCK) {
-        const int2 e = pairs[h];
-        if (e.x == 1) {
-            lo = min(lo, e.y);
-            hi = max(hi, e.y);
+    for (int64_t base = (int64_t)blockIdx.x * BLOCK * UNROLL; base < len;
+         base += (int64_t)gridDim.x * BLOCK * UNROLL) {
+        int2 e[UNROLL];
+#pragma unroll
+        for (int u = 0; u < UNROLL; u++) {
+            const int64_t h = base + u * BLOCK + threadIdx.x;
+            e[u] = h < len ? pairs[h] : make_int2(0, 0);
         }
+#pragma unroll
+        for (int u = 0; u < UNROLL; u++)
+            if (e[u].x == 1) {
+                lo = min(lo, e[u].y);
+                hi = max(hi, e[u].y);
+            }
     }
-    for (int off = 32; off > 0; off >>= 1) {
-        lo = min(lo, __shfl_xor(lo, off, 64));
-        hi = max(hi, __shfl_xor(hi, off, 64));
-    }
-    // one atomic pair per block: same-address atomics from every wave
-    // serialise in L2
-    __shared__ int32_t wlo[BLOCK / 64], whi[BLOCK / 64];
-    if ((threadIdx.x & 63) == 0) {
-        wlo[threadIdx.x >> 6] = lo;
-        whi[threadIdx.x >> 6] = hi;
-    }
-    __syncthreads();
+    block_minmax(lo, hi);
     if (threadIdx.x == 0) {
-        for (int w = 1; w < BLOCK / 64; w++) {
-            lo = min(lo, wlo[w]);
-            hi = max(hi, whi[w]);
-        }
-        if (lo <= hi) {
-            atomicMin(&info[0], lo);
-            atomicMax(&info[1], hi);
-        }
+        partials[2 * blockIdx.x] = lo;
+        partials[2 * blockIdx.x + 1] = hi;
     }
 }
 
-__global__ void __launch_bounds__(BLOCK) k_pairs_to_u16(const int2 *pairs, int64_t len, int32_t *info, uint16_t *u16)
+// The 16-bit copy and the presence bitmap of the pairs, 64 slots per wave and
+// step (a wave's ballot gives two bitmap words).  Every block first reduces
+// the partial ranges; block 0 leaves the result in info for the probe.
+__global__ void __launch_bounds__(BLOCK) k_pairs_to_u16(const int2 *__restrict__ pairs, int64_t len,
+                                                        const int32_t *__restrict__ partials, int nparts,
+                                                        int32_t *info, uint16_t *u16, uint32_t *bits)
 {
-    const int32_t vmin = info[0];
-    // every value offset must stay below VALS_UNSET
-    const bool fits = info[1] < info[0] || (int64_t)info[1] - (int64_t)vmin < (int64_t)VALS_UNSET;
-    if (!fits) {
-        if (blockIdx.x == 0 && threadIdx.x == 0) info[2] = 1;
-        return;
+    __shared__ int32_t range[2];
+    int32_t lo = INT32_MAX, hi = INT32_MIN;
+    if ((int)threadIdx.x < nparts) {
+        lo = partials[2 * threadIdx.x];
+        hi = partials[2 * threadIdx.x + 1];
     }
-    for (int64_t h = (int64_t)blockIdx.x * BLOCK + threadIdx.x; h < len; h += (int64_t)gridDim.x * BLOCK) {
-        const int2 e = pairs[h];
-        u16[h] = e.x == 1 ? (uint16_t)(e.y - vmin) : (uint16_t)VALS_UNSET;
+    block_minmax(lo, hi);
+    if (threadIdx.x == 0) {
+        range[0] = lo;
+        range[1] = hi;
+    }
+    __syncthreads();
+    const int32_t vmin = range[0];
+    // every value offset must stay below VALS_UNSET
+    const bool fits = range[1] < vmin || (int64_t)range[1] - (int64_t)vmin < (int64_t)VALS_UNSET;
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        info[0] = vmin;
+        info[1] = range[1];
+        info[2] = fits ? 0 : 1;
+    }
+    const int lane = threadIdx.x & 63;
+    const int64_t words = (len + 31) / 32, nwaves = (int64_t)gridDim.x * (BLOCK / 64);
+    for (int64_t g = (int64_t)blockIdx.x * (BLOCK / 64) + (threadIdx.x >> 6); g * 64 < len; g += nwaves) {
+        const int64_t h = g * 64 + lane;
+        const int2 e = h < len ? pairs[h] : make_int2(0, 0);
+        if (fits && h < len) u16[h] = e.x == 1 ? (uint16_t)(e.y - vmin) : (uint16_t)VALS_UNSET;
+        const uint64_t m = __ballot(e.x == 1);
+        if (lane < 2 && 2 * g + lane < words) bits[2 * g + lane] = (uint32_t)(m >> (32 * lane));
+    }
+}
+
+// The full probe of a long column against a table much smaller than it.  The
+// table's gathers are the bound: 268M of them into a 2.8 MB 16-bit table cost
+// 1.4 ms of 1.7 (each brings an L2 line for two bytes), against 0.35 ms for
+// the column and the flags.  So the block keeps in LDS (one 1024-thread block
+// per CU, 16 waves)
+//   VALS  the whole 16-bit table, up to PROBE_LDS_SLOTS slots;
+//   else  the presence bitmap, folded modulo the power of two that fits 128
+//         KB: a clear bit settles the row, and only the rows that pass (the
+//         matches and, folded, a few more) are listed and gather from the
+//         table, up to 256 of them in flight per wave.
+// 268M rows, 1.4M slots of which 4 % match, every row flagged: 1712 -> 712 us
+// (the scattered value stores are most of the rest); 60M rows, 300,000 slots,
+// 20 %: 374 -> 212 us; 61,130 slots in LDS, 0.8 % of 268M rows flagged: 340 ->
+// 237 us.  The column, flags and touched value lines alone take 600 / 180 /
+// 210 us at the rate of a copy.
+constexpr int PROBE_BLOCK = 1024;
+constexpr int64_t PROBE_LDS_SLOTS = 65536;        // 128 KB of 16-bit values
+constexpr uint32_t PROBE_FILTER_WORDS = 1u << 15; // 128 KB of presence bits
+constexpr int64_t PROBE_FILTER_SLOTS = 1 << 21;   // a listed row: slot and offset in its tile in 32 bits
+constexpr uint32_t PROBE_OFF_BITS = 11;
+static_assert(WT_ROWS == 1 << PROBE_OFF_BITS, "offset of a listed row");
+constexpr uint32_t PROBE_LIST_MIN = 256;          // listed rows per wave: a chunk of the tile at least
+constexpr uint32_t PROBE_LIST_MAX = 1024;
+constexpr int PROBE_DRAIN = 4;
+constexpr uint32_t PROBE_LDS_BYTES = 160 * 1024;
+
+// Listed rows per wave beside a filter of `fwords` words (and a row mask per lane)
+constexpr uint32_t probe_list_cap(uint32_t fwords)
+{
+    const uint32_t per_wave = (PROBE_LDS_BYTES - 4 * fwords) / 4 / (PROBE_BLOCK / 64) - 64;
+    return per_wave < PROBE_LIST_MAX ? per_wave : PROBE_LIST_MAX;
+}
+static_assert(probe_list_cap(PROBE_FILTER_WORDS) >= PROBE_LIST_MIN, "LDS of the largest filter and the lists");
+
+template <bool VALS>
+__global__ void __launch_bounds__(PROBE_BLOCK) k_probe_full_lds(const int32_t *__restrict__ probe, int32_t *val_out,
+                                                                const uint8_t *in, uint8_t *out, int64_t n,
+                                                                PairsOrU16 t, const uint32_t *__restrict__ bits,
+                                                                uint32_t words, uint32_t fwords, uint32_t cap,
+                                                                int32_t min, int32_t max)
+{
+    extern __shared__ uint4 probe_lds[];
+    const bool use16 = t.info[2] == 0;
+    const int32_t vmin = t.info[0];
+    const uint32_t span = (uint32_t)max - (uint32_t)min;
+    if constexpr (VALS) {
+        if (use16) // the 16-bit table (16-byte aligned and padded)
+            for (uint32_t i = threadIdx.x; i < (span + 8u) / 8u; i += PROBE_BLOCK)
+                probe_lds[i] = reinterpret_cast<const uint4 *>(t.u16)[i];
+    } else {
+        uint32_t *filter = reinterpret_cast<uint32_t *>(probe_lds);
+        for (uint32_t d = threadIdx.x; d < fwords; d += PROBE_BLOCK) {
+            uint32_t w = 0;
+            for (uint32_t k = d; k < words; k += fwords) w |= bits[k];
+            filter[d] = w;
+        }
+    }
+    __syncthreads();
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    // the wave's row masks and list, behind the filter
+    uint32_t *const hit_of = reinterpret_cast<uint32_t *>(probe_lds) + fwords + wave * (64 + cap);
+    uint32_t *const list = hit_of + 64;
+    const int64_t ntiles = (n + WT_ROWS - 1) / WT_ROWS, stride = (int64_t)gridDim.x * (PROBE_BLOCK / 64);
+    int64_t tile = (int64_t)blockIdx.x * (PROBE_BLOCK / 64) + wave;
+    uint32_t next[WT_CHUNKS];
+    if (tile < ntiles) wt_flags<true>(in, n, tile * WT_ROWS, lane, next);
+    for (; tile < ntiles; tile += stride) {
+        const int64_t t0 = tile * WT_ROWS;
+        const uint32_t flagged = wt_mask(next);
+        const bool whole = t0 + WT_ROWS <= n;
+        uint32_t slot[WT_CHUNKS][4];
+#pragma unroll
+        for (int j = 0; j < WT_CHUNKS; j++) {
+            const int64_t r = wt_row(t0, lane, j);
+            int4 x = make_int4(0, 0, 0, 0);
+            if ((flagged >> (4 * j)) & 15u) {
+                if (whole || r + 3 < n) x = *reinterpret_cast<const int4 *>(probe + r);
+                else {
+                    x.x = probe[r];
+                    if (r + 1 < n) x.y = probe[r + 1];
+                    if (r + 2 < n) x.z = probe[r + 2];
+                }
+            }
+            slot[j][0] = (uint32_t)x.x - (uint32_t)min;
+            slot[j][1] = (uint32_t)x.y - (uint32_t)min;
+            slot[j][2] = (uint32_t)x.z - (uint32_t)min;
+            slot[j][3] = (uint32_t)x.w - (uint32_t)min;
+        }
+        // the next tile's flags load while this one is probed
+        if (tile + stride < ntiles) wt_flags<true>(in, n, t0 + stride * WT_ROWS, lane, next);
+        uint32_t cand = 0;
+#pragma unroll
+        for (int b = 0; b < 4 * WT_CHUNKS; b++) {
+            const uint32_t s = slot[b >> 2][b & 3];
+            bool go = s <= span;
+            if constexpr (!VALS) {
+                const uint32_t *filter = reinterpret_cast<const uint32_t *>(probe_lds);
+                go &= ((filter[(s >> 5) & (fwords - 1)] >> (s & 31)) & 1u) != 0;
+            }
+            cand |= (uint32_t)go << b;
+        }
+        cand &= flagged;
+        uint32_t hits = 0;
+        if (!VALS && use16) {
+            if constexpr (!VALS) {
+                uint32_t total;
+                uint32_t at = wave_prefix((uint32_t)__popc(cand), lane, total);
+                hit_of[lane] = 0;
+                // a list too short for the tile takes a chunk (256 rows) at a time
+                const bool one = total <= cap;
+                uint32_t count = total;
+#pragma unroll
+                for (int j = 0; j < WT_CHUNKS; j++) {
+                    if (!one) at = wave_prefix((uint32_t)__popc((cand >> (4 * j)) & 15u), lane, count);
+#pragma unroll
+                    for (int k = 0; k < 4; k++)
+                        if ((cand >> (4 * j + k)) & 1u)
+                            list[at++] = slot[j][k] << PROBE_OFF_BITS | wt_offset(lane, 4 * j + k);
+                    if (one && j + 1 < WT_CHUNKS) continue;
+                    wave_sync();
+                    for (uint32_t e = 0; e < count; e += 64 * PROBE_DRAIN) {
+                        uint32_t v[PROBE_DRAIN], o[PROBE_DRAIN];
+#pragma unroll
+                        for (int d = 0; d < PROBE_DRAIN; d++) {
+                            const uint32_t i = e + 64 * d + lane;
+                            v[d] = VALS_UNSET;
+                            if (i < count) {
+                                o[d] = list[i];
+                                v[d] = t.u16[o[d] >> PROBE_OFF_BITS];
+                            }
+                        }
+#pragma unroll
+                        for (int d = 0; d < PROBE_DRAIN; d++) {
+                            if (v[d] == VALS_UNSET) continue;
+                            o[d] &= (1u << PROBE_OFF_BITS) - 1;
+                            val_out[t0 + o[d]] = vmin + (int32_t)v[d];
+                            atomicOr(&hit_of[(o[d] >> 2) & 63u], 1u << ((o[d] >> 8) * 4 + (o[d] & 3u)));
+                        }
+                    }
+                    wave_sync();
+                }
+                hits = hit_of[lane];
+                wave_sync();
+            }
+        } else {
+#pragma unroll
+            for (int j = 0; j < WT_CHUNKS; j++) {
+                if (!((cand >> (4 * j)) & 15u)) continue;
+                const int64_t r = wt_row(t0, lane, j);
+                int32_t v[4];
+                uint32_t hit = 0;
+#pragma unroll
+                for (int k = 0; k < 4; k++) {
+                    if (!((cand >> (4 * j + k)) & 1u)) continue;
+                    if (VALS && use16) {
+                        const uint32_t raw = reinterpret_cast<const uint16_t *>(probe_lds)[slot[j][k]];
+                        v[k] = vmin + (int32_t)raw;
+                        hit |= (uint32_t)(raw != VALS_UNSET) << k;
+                    } else {
+                        const int2 e = t.pairs[slot[j][k]];
+                        v[k] = e.y;
+                        hit |= (uint32_t)(e.x == 1) << k;
+                    }
+                }
+#pragma unroll
+                for (int k = 0; k < 4; k++)
+                    if ((hit >> k) & 1u) val_out[r + k] = v[k];
+                hits |= hit << (4 * j);
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < WT_CHUNKS; j++) {
+            const int64_t r = wt_row(t0, lane, j);
+            const uint32_t f = flag_bytes(hits >> (4 * j));
+            if (whole || r + 3 < n) *reinterpret_cast<uint32_t *>(out + r) = f;
+            else
+                for (int k = 0; k < 4; k++)
+                    if (r + k < n) out[r + k] = (uint8_t)(f >> (8 * k));
+        }
     }
 }
 
@@ -520,19 +799,6 @@ __device__ __forceinline__ uint64_t wave_sum_u64(uint64_t v)
     for (int off = 32; off > 0; off >>= 1)
         v += __shfl_xor(v, off, 64);
     return v;
-}
-
-// Exclusive prefix of v over the lanes of the wave, and the total.
-__device__ __forceinline__ uint32_t wave_prefix(uint32_t v, int lane, uint32_t &total)
-{
-    uint32_t x = v;
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-        const uint32_t y = __shfl_up(x, off, 64);
-        if (lane >= off) x += y;
-    }
-    total = __builtin_amdgcn_readlane(x, 63);
-    return x - v;
 }
 
 // The scalar reductions run 1024-thread blocks, at most two per CU: each block
@@ -635,56 +901,6 @@ struct GroupArgs {
     uint32_t range[GB_MAX_KEYS]; // max - min + 1 (uint32 image of the int)
     int k;
 };
-
-// Tiles of WT_ROWS rows per wave: chunk j of a lane holds the rows
-// t0 + 256 j + 4 lane .. + 3, so that flags (4 bytes) and columns (16 bytes)
-// load coalesced; bit 4 j + k of a lane's 32-bit row mask is row k of its
-// chunk j.
-constexpr int WT_CHUNKS = 8;
-constexpr int64_t WT_ROWS = 256 * WT_CHUNKS;
-
-__device__ __forceinline__ int64_t wt_row(int64_t t0, int lane, int j) { return t0 + 256 * j + 4 * lane; }
-// offset in its tile of the row of mask bit b
-__device__ __forceinline__ uint32_t wt_offset(int lane, uint32_t b) { return (b >> 2) * 256u + 4u * lane + (b & 3u); }
-
-// Flags of a tile (rows at or past n: 0).  VEC: flags 4-byte aligned.
-template <bool VEC>
-__device__ __forceinline__ void wt_flags(const uint8_t *flags, int64_t n, int64_t t0, int lane, uint32_t (&f)[WT_CHUNKS])
-{
-    if (VEC && t0 + WT_ROWS <= n) {
-#pragma unroll
-        for (int j = 0; j < WT_CHUNKS; j++) f[j] = *reinterpret_cast<const uint32_t *>(flags + wt_row(t0, lane, j));
-        return;
-    }
-#pragma unroll
-    for (int j = 0; j < WT_CHUNKS; j++) {
-        const int64_t r = wt_row(t0, lane, j);
-        f[j] = 0;
-#pragma unroll
-        for (int k = 0; k < 4; k++)
-            if (r + k < n) f[j] |= (uint32_t)flags[r + k] << (8 * k);
-    }
-}
-
-// Bit k: whether byte k of x is nonzero (the flag bits 0, 8, 16, 24 of
-// nz_bytes meet in bits 24..27 of the product, with no carry into them).
-__device__ __forceinline__ uint32_t nz_mask(uint32_t x) { return (nz_bytes(x) * 0x01020408u) >> 24; }
-
-__device__ __forceinline__ uint32_t wt_mask(const uint32_t (&f)[WT_CHUNKS])
-{
-    uint32_t m = 0;
-#pragma unroll
-    for (int j = 0; j < WT_CHUNKS; j++) m |= nz_mask(f[j]) << (4 * j);
-    return m;
-}
-
-// LDS written by some lanes of a wave and read by others
-__device__ __forceinline__ void wave_sync()
-{
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
 
 // Dense slot of row i exactly as GroupByAggregateKernel computes it
 // (int32 wrapping accumulation, then % prod on the uint64 image).
@@ -1563,15 +1779,38 @@ void launch_probe_full(const int32_t *probe, int32_t *val_out, const uint8_t *in
     // instead of 8)
     const int64_t len = max >= min ? (int64_t)max - min + 1 : 0;
     if (n >= PROBE_U16_MIN_ROWS && len > 0 && len * PROBE_U16_MIN_RATIO <= n && len <= PROBE_U16_MAX_SLOTS) {
-        uint8_t *scr = static_cast<uint8_t *>(scratch_buffer(256 + (size_t)len * 2, s));
+        const size_t words = (size_t)((len + 31) / 32), part_off = 256;
+        const size_t u16_off = part_off + PAIRS_RANGE_BLOCKS * 8, bits_off = u16_off + ((size_t)len * 2 + 15) / 16 * 16;
+        uint8_t *scr = static_cast<uint8_t *>(scratch_buffer(bits_off + words * 4, s));
         int32_t *info = reinterpret_cast<int32_t *>(scr);
-        uint16_t *u16 = reinterpret_cast<uint16_t *>(scr + 256);
+        int32_t *partials = reinterpret_cast<int32_t *>(scr + part_off);
+        uint16_t *u16 = reinterpret_cast<uint16_t *>(scr + u16_off);
+        uint32_t *bits = reinterpret_cast<uint32_t *>(scr + bits_off);
+        const unsigned gr =
+            (unsigned)std::min<int64_t>((len + BLOCK * UNROLL - 1) / (BLOCK * UNROLL), PAIRS_RANGE_BLOCKS);
         const unsigned g = (unsigned)std::min<int64_t>((len + BLOCK - 1) / BLOCK, 1024);
-        hipLaunchKernelGGL(k_pairs_range_init, dim3(1), dim3(1), 0, s, info);
-        hipLaunchKernelGGL(k_pairs_range, dim3(g), dim3(BLOCK), 0, s, t.pairs, len, info);
-        hipLaunchKernelGGL(k_pairs_to_u16, dim3(g), dim3(BLOCK), 0, s, t.pairs, len, info, u16);
+        hipLaunchKernelGGL(k_pairs_range, dim3(gr), dim3(BLOCK), 0, s, t.pairs, len, partials);
+        hipLaunchKernelGGL(k_pairs_to_u16, dim3(g), dim3(BLOCK), 0, s, t.pairs, len, partials, (int)gr, info, u16, bits);
         t.u16 = u16;
         t.info = info;
+        const dim3 grid(stream_grid(n, WT_ROWS * (PROBE_BLOCK / 64), 1));
+        if (vec && len <= PROBE_LDS_SLOTS) {
+            const size_t lds = ((size_t)len * 2 + 15) / 16 * 16;
+            hipLaunchKernelGGL((k_probe_full_lds<true>), grid, dim3(PROBE_BLOCK), lds, s, probe, val_out, in, out, n, t,
+                               bits, (uint32_t)words, 0u, 0u, min, max);
+            check_launch("probe_full");
+            return;
+        }
+        if (vec && len <= PROBE_FILTER_SLOTS) {
+            uint32_t fwords = 1;
+            while (fwords < words && fwords < PROBE_FILTER_WORDS) fwords *= 2;
+            const uint32_t cap = probe_list_cap(fwords);
+            const size_t lds = ((size_t)fwords + (PROBE_BLOCK / 64) * (64 + cap)) * 4;
+            hipLaunchKernelGGL((k_probe_full_lds<false>), grid, dim3(PROBE_BLOCK), lds, s, probe, val_out, in, out, n, t,
+                               bits, (uint32_t)words, fwords, cap, min, max);
+            check_launch("probe_full");
+            return;
+        }
     }
     hipLaunchKernelGGL(k_probe_full, dim3(vec ? grid_rows(n) : grid_one(n)), dim3(BLOCK), 0, s, probe, val_out, in,
                        out, n, t, min, max, vec);

@@ -106,3 +106,49 @@ def test_groupby_lds_largest_range(ops):
         want = np.bincount(key[fl != 0], weights=agg[fl != 0], minlength=prod).astype(np.int64)
         assert (sums.cpu().numpy() == want).all()
         assert ((seen.cpu().numpy() != 0) == (np.bincount(key[fl != 0], minlength=prod) > 0)).all()
+
+
+# Probes over at least 4M rows and 16 rows per table slot: the 16-bit table in
+# LDS up to 65,536 slots; the presence bitmap in LDS, whole up to 2^20 slots,
+# folded above; few matches (listed) and many (gathered where they lie), few
+# and many flagged rows; values too wide for 16 bits; in place; a ragged end.
+@pytest.mark.parametrize("length,match,flagged,wide", [
+    (1, 1.0, 1.0, False), (61_130, 0.04, 0.01, False), (65_536, 1.0, 0.5, False), (65_536, 0.5, 1.0, True),
+    (65_537, 0.03, 1.0, False), (65_537, 0.9, 0.3, True), (300_000, 0.2, 0.02, False), (280_001, 0.0, 1.0, False)])
+def test_probe_full_lds_tables(ops, length, match, flagged, wide):
+    import torch
+    rng = np.random.default_rng(length)
+    n, mn = 4_500_003, -1000
+    mx = mn + length - 1
+    pairs = np.zeros(2 * length, np.int32)
+    pairs[0::2] = np.where(rng.random(length) < match, 1, rng.integers(0, 2, length) * 2)  # 2 is no match
+    pairs[1::2] = rng.integers(-5, 65_529 if not wide else 2**31, length)
+    probe = rng.integers(mn - length // 8 - 1, mx + length // 8 + 2, n).astype(np.int32)
+    probe[:3] = [-2**31, 2**31 - 1, mx]
+    fl = flags_of(rng, n, flagged)
+    tf, vo = dev(fl), torch.full((n,), -77, dtype=torch.int32, device="cuda")
+    ops.full_join(dev(probe), vo, tf, n, dev(pairs), mn, mx)
+    want, want_v = np.zeros(n, np.uint8), np.full(n, -77, np.int32)
+    O.probe_full(probe, want_v, fl, want, pairs, mn, mx)
+    assert (tf.cpu().numpy() == want).all() and (vo.cpu().numpy() == want_v).all()
+
+
+@pytest.mark.parametrize("length,match", [(1_400_000, 0.04), (1_400_000, 0.7), (2_097_152, 0.01), (2_097_153, 0.01)])
+def test_probe_full_folded_filter(ops, length, match):
+    """Tables of more slots than the filter has bits, up to its largest fold
+    and one slot past it (no filter)."""
+    import torch
+    g = torch.Generator("cuda").manual_seed(length)
+    n, mn = 16 * length + 5, 7
+    pairs = torch.zeros(2 * length, dtype=torch.int32, device="cuda")
+    pairs[0::2] = (torch.rand(length, generator=g, device="cuda") < match).int()
+    pairs[1::2] = torch.randint(100, 1100, (length,), generator=g, device="cuda", dtype=torch.int32)
+    probe = torch.randint(mn - 50, mn + length + 50, (n,), generator=g, device="cuda", dtype=torch.int32)
+    fl = (torch.rand(n, generator=g, device="cuda") < 0.9).to(torch.uint8)
+    out, vo = torch.full((n,), 9, dtype=torch.uint8, device="cuda"), torch.full((n,), -7, dtype=torch.int32, device="cuda")
+    ops.probe_full(probe, vo, fl, out, pairs, mn, mn + length - 1)
+    s = probe - mn
+    inside = (s >= 0) & (s < length)
+    s = torch.where(inside, s, 0).long()
+    hit = (fl != 0) & inside & (pairs[0::2][s] == 1)
+    assert bool((out == hit).all()) and bool((vo == torch.where(hit, pairs[1::2][s], -7)).all())
