@@ -264,8 +264,7 @@ struct Staging {
 
 uint32_t bitmap_stage_bytes(const FInstr &I)
 {
-    const uint64_t len = (uint64_t)((int64_t)I.ht_max - I.ht_min + 1);
-    return (uint32_t)(((len + 31) / 32 + 3) / 4 * 16);
+    return (uint32_t)bitmap_bytes16((uint64_t)((int64_t)I.ht_max - I.ht_min + 1));
 }
 
 bool is_predicate(uint8_t k)
@@ -484,6 +483,44 @@ double prefetch_min_touch()
         return e && *e ? atof(e) : 0.3;
     }();
     return v;
+}
+
+// The probe that gets a presence filter in LDS (-1: none): the first bitmap
+// probe in global memory that few rows pass.  Its table is then read for
+// those rows alone (and those the fold lets through), not for every row that
+// reaches it.  q2.x at 600M rows
+// (part: 1.4M slots, 4 % set, 20 % of the rows reach it): the kernel 1395 ->
+// 1012 us, 0.2 of its 16-bit table reads left.  The line: a table of 2^20
+// slots or more, whose 16-bit values take half of an XCD's L2 (300,000 slots:
+// 224 us without, 231 with); 2^25 rows, whose saved reads pay for staging the
+// filter in every block (about 10 us); at most 30 % of the rows passing.
+// SDB_FOLD_FILTER=0 turns it off.
+constexpr int64_t FOLD_MIN_ROWS = 32 << 20;
+constexpr double FOLD_MIN_SLOTS = 1 << 20;
+constexpr double FOLD_MAX_PASS = 0.3, FOLD_MIN_LIVE = 0.1;
+
+int choose_fold(const std::vector<Draft> &d, const std::vector<Staging> &st, int64_t n)
+{
+    static const bool on = [] {
+        const char *e = getenv("SDB_FOLD_FILTER");
+        return !(e && *e == '0');
+    }();
+    if (!on || n < FOLD_MIN_ROWS) return -1;
+    double live = 1.0;
+    for (size_t i = 0; i < d.size(); i++) {
+        const FInstr &I = d[i].I;
+        if (!is_predicate(I.kind)) continue;
+        if (!is_conjunctive(I)) return -1;
+        if (I.kind == FK_PROBE_BITS && !st[i].src) {
+            if ((double)I.ht_max - I.ht_min + 1 < FOLD_MIN_SLOTS) return -1;
+            const double bits = 8.0 * std::min<double>(F_FOLD_MAX, bitmap_stage_bytes(I));
+            const double fold = std::max(1.0, ((double)I.ht_max - I.ht_min + 1) / bits);
+            const double pass = 1.0 - std::pow(1.0 - std::min(1.0, std::max(0.0, (double)d[i].sel)), fold);
+            return pass <= FOLD_MAX_PASS && live >= FOLD_MIN_LIVE && I.va >= F_PF_BASE ? (int)i : -1;
+        }
+        live *= std::max(0.0f, std::min(1.0f, d[i].sel));
+    }
+    return -1;
 }
 
 void assign_prefetch(std::vector<Draft> &d, FGroup &g, FProgram &p)
@@ -956,6 +993,14 @@ bool KernelBundle::build_program(const ExecContext &ctx, FProgram &p) const
                 I.vals = nullptr;
                 I.ht_len = (int32_t)((((int64_t)I.ht_max - I.ht_min + 1) + 31) / 32);
             }
+        }
+        // an explicit launch shape keeps its small blocks, several per CU
+        const int f = captured || eng.unroll || eng.codegen == SDB_CODEGEN_INTERPRET ? -1 : choose_fold(d, st, n);
+        if (f >= 0) {
+            p.fold = (uint32_t)f + 1;
+            p.fold_total = bitmap_stage_bytes(p.ins[f]);
+            p.fold_bytes = 16;
+            while (p.fold_bytes < p.fold_total && p.fold_bytes < F_FOLD_MAX) p.fold_bytes *= 2;
         }
     }
     if (p.gb.lds == FG_DENSE_LDS) {

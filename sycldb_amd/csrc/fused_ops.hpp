@@ -224,6 +224,46 @@ __device__ __forceinline__ uint32_t probe_bits_finish(const int32_t (&x)[R], uin
     return out;
 }
 
+// The rows of `in` whose key may be in a probe's table: its presence bitmap,
+// folded modulo `mask` + 1 words, in LDS (a clear bit is certain).
+template <int R>
+__device__ __forceinline__ uint32_t fold_pass(const int32_t (&x)[R], uint32_t in, const uint32_t *filter, uint32_t mask,
+                                              int32_t mn, int32_t mx)
+{
+    const uint32_t span = (uint32_t)mx - (uint32_t)mn;
+    uint32_t out = 0;
+#pragma unroll
+    for (int k = 0; k < R; k++) {
+        const uint32_t s = (uint32_t)x[k] - (uint32_t)mn;
+        out |= (uint32_t)((s <= span) & (((filter[(s >> 5) & mask] >> (s & 31)) & 1u) != 0)) << k;
+    }
+    return mx >= mn ? out & in : 0u;
+}
+
+// Where the compiled kernel keeps that filter, and its staging at block start.
+__device__ __forceinline__ uint32_t *fold_filter(const FProgram &P, uint8_t *lds)
+{
+    return reinterpret_cast<uint32_t *>(lds + ((P.vreg_off + 15u) & ~15u));
+}
+
+template <int NT> __device__ __forceinline__ void fold_stage(const FProgram &P, uint8_t *lds)
+{
+    const uint4 *src = reinterpret_cast<const uint4 *>(P.ins[P.fold - 1].ht);
+    uint4 *dst = reinterpret_cast<uint4 *>(fold_filter(P, lds));
+    const uint32_t n = P.fold_bytes / 16, total = P.fold_total / 16;
+    for (uint32_t d = threadIdx.x; d < n; d += NT) {
+        uint4 w = make_uint4(0u, 0u, 0u, 0u);
+        for (uint32_t k = d; k < total; k += n) {
+            const uint4 q = src[k];
+            w.x |= q.x;
+            w.y |= q.y;
+            w.z |= q.z;
+            w.w |= q.w;
+        }
+        dst[d] = w;
+    }
+}
+
 // A bitmap probe answered by its FV_U16 value table alone: a slot reads
 // VALS_UNSET exactly when its presence bit is clear, so one read gives both
 // the match and the value (no bitmap read).  Rows outside the key range or

@@ -133,6 +133,12 @@ struct FProgram {
     const void *blob_src[F_MAX_BLOBS];
     uint32_t blob_bytes[F_MAX_BLOBS]; // multiples of 16
     uint32_t blob_off[F_MAX_BLOBS];
+    // Presence filter of a compiled kernel (the interpreter does without):
+    // instruction fold - 1, a bitmap probe in global memory, first tests its
+    // keys against its bitmap folded modulo fold_bytes (a power of two) in
+    // LDS; only rows that pass read the table.  fold_total: bitmap bytes,
+    // padded to 16.  0: no filter.
+    uint32_t fold, fold_bytes, fold_total;
     uint8_t flag_init[F_MAX_FLAGS];
     const uint8_t *flag_load[F_MAX_FLAGS];
     uint8_t *flag_store[F_MAX_FLAGS];
@@ -199,8 +205,14 @@ __host__ __device__ constexpr uint32_t dict_vals_off(uint32_t len) { return (6u 
 // bytes of the LDS part with room for F_DICT_CAP windows
 __host__ __device__ constexpr uint32_t dict_lds_bytes(uint32_t len) { return dict_vals_off(len) + 4u * F_DICT_CAP; }
 
+// Bytes of a presence bitmap over len slots, padded to 16.
+__host__ __device__ constexpr uint64_t bitmap_bytes16(uint64_t len) { return ((len + 31) / 32 + 3) / 4 * 16; }
+
 // Largest rank dictionary built for LDS staging.
 constexpr uint32_t F_RANK_DICT_MAX = 32 * 1024;
+
+// LDS of a compiled kernel's presence filter at most.
+constexpr uint32_t F_FOLD_MAX = 64 * 1024;
 
 // Dynamic LDS one fused block may use (registers, staged bitmaps, group-by).
 constexpr uint32_t F_LDS_BUDGET = 96 * 1024;

@@ -136,6 +136,10 @@ struct Gen {
     std::vector<bool> decided;
     explicit Gen(const FProgram &prog, bool prefetch = true) : p(prog), prefetch_in_body(prefetch) {}
 
+    bool folded(int i) const { return !batch_act && p.fold == (uint32_t)i + 1; }
+    // the rows a folded probe reads its table for
+    static std::string fold_reg(int i) { return "fold" + std::to_string(i) + "[u]"; }
+
     bool is_decided(int i) const { return i < (int)decided.size() && decided[i]; }
     bool dropped(int i) const
     {
@@ -260,7 +264,7 @@ struct Gen {
 
     // Load phase of probe i (operand rows into x<i>, table reads into t<i>)
     // for the rows of flag mask `gate`.
-    std::string probe_issue(int i, const std::string &gate) const
+    std::string probe_issue(int i, const std::string &in) const
     {
         const FInstr &I = p.ins[i];
         const std::string P = "P.ins[" + std::to_string(i) + "]";
@@ -268,7 +272,11 @@ struct Gen {
         const std::string U = "#pragma unroll\n        for (int u = 0; u < UU; u++) ";
         std::ostringstream a;
         if (cheap(I.va)) a << U << "{ " << operand(I.va, P + ".a", x) << " }\n";
-        else a << U << "if (" << gate << ") { " << operand(I.va, P + ".a", x) << " }\n";
+        else a << U << "if (" << in << ") { " << operand(I.va, P + ".a", x) << " }\n";
+        const std::string gate = folded(i) ? fold_reg(i) : in;
+        if (folded(i))
+            a << U << gate << " = " << in << " ? fold_pass<R>(" << x << ", " << in << ", fold_filter(P, lds), P.fold_bytes / 4 - 1, "
+              << P << ".ht_min, " << P << ".ht_max) : 0u;\n";
         a << U << "if (" << gate << ") ";
         if (is_decided(i)) {
             // the value alone (FV_U16 / FV_PAIR tables, or the reference pairs)
@@ -477,6 +485,7 @@ struct Gen {
                 c << "            " << fout << " = o;\n        }\n";
                 break;
             }
+            const std::string fin = folded(i) ? fold_reg(i) : freg(I.fin) + "[u]";
             c << U << "{\n            uint32_t o = 0;\n";
             if (!vout || late_value(i)) c << "            int32_t none[R];\n";
             c << "            if (" << fin << ") {\n";
@@ -862,7 +871,7 @@ struct Gen {
            << "    __builtin_amdgcn_wave_barrier();\n"
            << "    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, \"wavefront\");\n}\n";
         fn << "__device__ __forceinline__ int32_t *queue_base(const FProgram &P, uint8_t *lds)\n{\n"
-           << "    return reinterpret_cast<int32_t *>(lds + ((P.vreg_off + 15u) & ~15u)) + (threadIdx.x >> 6) * (64 * QF);\n}\n"
+           << "    return reinterpret_cast<int32_t *>(lds + ((P.vreg_off + 15u) & ~15u) + P.fold_bytes) + (threadIdx.x >> 6) * (64 * QF);\n}\n"
            << "__device__ __forceinline__ void queue_flush(const FProgram &P, uint8_t *lds, int64_t &acc, uint32_t &qn)\n{\n"
            << "    int32_t *const qb = queue_base(P, lds);\n    wave_sync();\n"
            << "    const uint32_t lane = threadIdx.x & 63u;\n    if (lane < qn) {\n"
@@ -941,7 +950,8 @@ struct Gen {
         const int dense_end = tail_start >= 0 ? tail_start : p.ninstr;
         for (int i = 0; i < dense_end; i++)
             if (is_probe(p.ins[i].kind) && !dropped(i))
-                o << "    int32_t x" << i << "[UU][R];\n    ProbeTmp<R> t" << i << "[UU];\n";
+                o << "    int32_t x" << i << "[UU][R];\n    ProbeTmp<R> t" << i << "[UU];\n"
+                  << (folded(i) ? "    uint32_t fold" + std::to_string(i) + "[UU];\n" : std::string());
         // the next tile's column loads go out after the loads of the first
         // instruction that waits for global memory and before that wait, so
         // the in-order completion counter does not make it wait for them too
@@ -1010,6 +1020,7 @@ extern "C" __global__ void __launch_bounds__(BLOCK) sdb_fused_program(const FPro
     if (P.magic != F_MAGIC) return;
     extern __shared__ uint4 dyn_lds[];
     uint8_t *lds = reinterpret_cast<uint8_t *>(dyn_lds);
+    if constexpr (FOLD) fold_stage<BLOCK>(P, lds);
     fdev::block_prologue<BLOCK>(P, lds);
     int64_t acc = 0;
     uint32_t qn = 0; // rows in this wave's queue (queued tail)
@@ -1271,6 +1282,8 @@ std::vector<std::pair<FProgram, int>> coverage_programs()
         p.gb.lds = FG_HASH_LDS;
         p.gb.key_reg[0] = 1, p.gb.key_reg[1] = 0;
         p.gb.agg_reg = F_PF_BASE + 3;
+        p.fold = 2; // the global probe behind a presence filter in LDS
+        p.fold_bytes = F_FOLD_MAX;
         out.emplace_back(p, 2);
     }
     {   // star join whose later columns are read from memory: the date key
@@ -1420,6 +1433,7 @@ std::string shape_key(const FProgram &p)
     put(p.vec);
     put(p.nvals);
     put(p.npf);
+    put((int)p.fold);
     for (int j = 0; j < F_MAX_FLAGS; j++) {
         put(p.flag_init[j]);
         put(p.flag_load[j] != nullptr);
@@ -1488,6 +1502,7 @@ std::string jit_source(const FProgram &p, int unroll, int block, bool queue)
     std::ostringstream s;
     s << KERNEL_TEMPLATE_INCLUDES << "constexpr int NPF = " << p.npf << ";\nconstexpr int U = " << unroll
       << ";\nconstexpr bool VEC = " << (p.vec ? "true" : "false") << ";\nconstexpr int BLOCK = " << block << ";\n";
+    s << "constexpr bool FOLD = " << (p.fold ? "true" : "false") << ";\n";
     s << "constexpr bool QUEUE = " << (g.queue ? "true" : "false") << ";\nconstexpr int QF = " << g.queue_fields
       << ";\n";
     s << (g.queue ? g.queue_fn : std::string(KERNEL_QUEUE_STUB));
@@ -1526,6 +1541,8 @@ Compiled &kernel_for(const FProgram &p, int unroll, int block, bool queue, uint3
 // Largest dynamic LDS of a launch with a row queue; past it (or past 2^31
 // rows, whose indices the queue does not hold) the kernel without one runs.
 constexpr uint64_t QUEUE_LDS_MAX = 96 * 1024;
+// The same beside a presence filter, which leaves one block per CU anyway.
+constexpr uint64_t FOLD_LDS_MAX = 156 * 1024;
 
 // The kernel a launch of n rows uses (with a row queue when `queue` allows
 // one and it fits), its dynamic LDS bytes, and whether it has the queue.
@@ -1533,19 +1550,20 @@ Compiled &pick_kernel(const FProgram &p, int64_t n, int unroll, int block, bool 
                       bool *queued = nullptr)
 {
     uint32_t qbytes = 0;
+    const uint32_t fixed = p.fold ? (p.vreg_off + 15u) / 16u * 16u + p.fold_bytes : p.vreg_off;
     if (queued) *queued = false;
     if (queue && n <= INT32_MAX) {
         Compiled &k = kernel_for(p, unroll, block, true, &qbytes);
         // the value-register file (the last LDS area) belongs to the
         // interpreter; the queues of the block's waves go there instead
-        const uint64_t total = ((uint64_t)p.vreg_off + 15u) / 16u * 16u + (uint64_t)(block / 64) * qbytes;
-        if (!qbytes || total <= QUEUE_LDS_MAX) {
-            lds = qbytes ? (uint32_t)total : p.vreg_off;
+        const uint64_t total = fixed + (uint64_t)(block / 64) * qbytes;
+        if (!qbytes || total <= (p.fold ? FOLD_LDS_MAX : QUEUE_LDS_MAX)) {
+            lds = qbytes ? (uint32_t)total : fixed;
             if (queued) *queued = qbytes != 0;
             return k;
         }
     }
-    lds = p.vreg_off;
+    lds = fixed;
     return kernel_for(p, unroll, block, false, &qbytes);
 }
 

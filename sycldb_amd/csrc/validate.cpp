@@ -272,6 +272,15 @@ void validate_program(const FProgram &p, int64_t n_rows, const AllocRegistry &re
         default: fail(SDB_ERR_RUNTIME, "launch check: unknown instruction");
         }
     }
+    if (p.fold) {
+        if (p.fold > (uint32_t)p.ninstr || (p.fold_bytes & (p.fold_bytes - 1)) || p.fold_bytes < 16 ||
+            p.fold_bytes > F_FOLD_MAX || p.vreg_off > F_LDS_BUDGET)
+            fail(SDB_ERR_RUNTIME, "launch check: presence filter size");
+        const FInstr &I = p.ins[p.fold - 1];
+        if (I.kind != FK_PROBE_BITS || I.in_lds || p.fold_total != bitmap_bytes16(range_len(I.ht_min, I.ht_max)))
+            fail(SDB_ERR_RUNTIME, "launch check: presence filter probe");
+        reg.check(I.ht, p.fold_total, "presence filter bitmap");
+    }
     if (p.sum_acc && !has_sum) fail(SDB_ERR_RUNTIME, "launch check: accumulator without sum");
     if (p.gb.prod && !has_gb) fail(SDB_ERR_RUNTIME, "launch check: group spec without group-by");
 }
