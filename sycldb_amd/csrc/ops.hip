@@ -22,6 +22,7 @@ namespace {
 
 constexpr int BLOCK = 256;
 constexpr int UNROLL = 4;
+constexpr uint32_t LDS_PER_CU = 160 * 1024; // gfx950
 constexpr int64_t ROWS_PER_STEP = (int64_t)BLOCK * UNROLL * 4;
 
 inline bool aligned(const void *p, size_t a) { return ((uintptr_t)p % a) == 0; }
@@ -325,6 +326,10 @@ __device__ __forceinline__ uint32_t wt_mask(const uint32_t (&f)[WT_CHUNKS])
     return m;
 }
 
+// The wave's index in its block, in a scalar register: addresses that follow
+// from it (a tile's) then are scalar bases with 32-bit offsets per lane.
+__device__ __forceinline__ int wave_index() { return __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); }
+
 // LDS written by some lanes of a wave and read by others
 __device__ __forceinline__ void wave_sync()
 {
@@ -442,6 +447,74 @@ __global__ void __launch_bounds__(BLOCK) k_probe_semi(const int32_t *__restrict_
         bool r = false;
         if (f) r = present(probe[i]);
         out[i] = r;
+    }
+}
+
+// The semi probe of a long column.  The kernel above waits for each flagged
+// row's table byte in turn, up to 16 round trips to L2 per step of a thread.
+// Here a block first turns the table into a bitmap in LDS, one bit per slot,
+// and the 16 answers of a step are read without a branch; two 1024-thread
+// blocks per CU.  200M rows (the column and the flags alone take 228 us, what
+// select_lit measures): 20,000 slots, every row flagged 381 -> 234 us, one in
+// five 288 -> 235; 300,000 slots 345 -> 243; 61,130 slots, 5 % flagged 277 -> 236.
+constexpr int SEMI_BLOCK = 1024;
+
+__global__ void __launch_bounds__(SEMI_BLOCK) k_probe_semi_lds(const int32_t *__restrict__ probe, const uint8_t *in,
+                                                               uint8_t *out, int64_t n, const uint8_t *__restrict__ ht,
+                                                               uint32_t slots, int32_t min)
+{
+    extern __shared__ uint4 semi_lds[];
+    uint16_t *const half = reinterpret_cast<uint16_t *>(semi_lds);
+    for (uint32_t h = threadIdx.x; h < (slots + 15u) / 16u; h += SEMI_BLOCK) {
+        uint32_t w[4] = {0, 0, 0, 0};
+        if (16u * h + 16u <= slots) {
+            const uint4 q = reinterpret_cast<const uint4 *>(ht)[h];
+            w[0] = q.x;
+            w[1] = q.y;
+            w[2] = q.z;
+            w[3] = q.w;
+        } else {
+#pragma unroll
+            for (uint32_t k = 0; k < 16u; k++)
+                if (16u * h + k < slots) w[k >> 2] |= (uint32_t)ht[16u * h + k] << (8u * (k & 3u));
+        }
+        half[h] = (uint16_t)(nz_mask(w[0]) | nz_mask(w[1]) << 4 | nz_mask(w[2]) << 8 | nz_mask(w[3]) << 12);
+    }
+    __syncthreads();
+    const uint32_t *const bits = reinterpret_cast<const uint32_t *>(semi_lds);
+    const uint32_t last = (slots - 1u) >> 5;
+    const int64_t nchunks = n >> 2;
+    const int4 *p4 = reinterpret_cast<const int4 *>(probe);
+    const uint32_t *in32 = reinterpret_cast<const uint32_t *>(in);
+    uint32_t *out32 = reinterpret_cast<uint32_t *>(out);
+    for (int64_t base = (int64_t)blockIdx.x * SEMI_BLOCK * UNROLL; base < nchunks;
+         base += (int64_t)gridDim.x * SEMI_BLOCK * UNROLL) {
+        uint32_t f[UNROLL];
+        int4 x[UNROLL];
+#pragma unroll
+        for (int u = 0; u < UNROLL; u++) {
+            const int64_t c = base + u * SEMI_BLOCK + threadIdx.x;
+            f[u] = c < nchunks ? in32[c] : 0u;
+            x[u] = c < nchunks ? p4[c] : make_int4(0, 0, 0, 0);
+        }
+#pragma unroll
+        for (int u = 0; u < UNROLL; u++) {
+            const int64_t c = base + u * SEMI_BLOCK + threadIdx.x;
+            const int32_t xs[4] = {x[u].x, x[u].y, x[u].z, x[u].w};
+            uint32_t hit = 0;
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                const uint32_t s = (uint32_t)xs[k] - (uint32_t)min;
+                const uint32_t w = bits[::min(s >> 5, last)]; // past the table: any word
+                hit |= (uint32_t)(s < slots && ((w >> (s & 31u)) & 1u)) << k;
+            }
+            if (c < nchunks) out32[c] = flag_bytes(hit & nz_mask(f[u]));
+        }
+    }
+    if (blockIdx.x == 0 && threadIdx.x < (n & 3)) {
+        const int64_t i = (nchunks << 2) + threadIdx.x;
+        const uint32_t s = (uint32_t)probe[i] - (uint32_t)min;
+        out[i] = in[i] && s < slots && ht[s] != 0;
     }
 }
 
@@ -633,12 +706,11 @@ static_assert(WT_ROWS == 1 << PROBE_OFF_BITS, "offset of a listed row");
 constexpr uint32_t PROBE_LIST_MIN = 256;          // listed rows per wave: a chunk of the tile at least
 constexpr uint32_t PROBE_LIST_MAX = 1024;
 constexpr int PROBE_DRAIN = 4;
-constexpr uint32_t PROBE_LDS_BYTES = 160 * 1024;
 
 // Listed rows per wave beside a filter of `fwords` words (and a row mask per lane)
 constexpr uint32_t probe_list_cap(uint32_t fwords)
 {
-    const uint32_t per_wave = (PROBE_LDS_BYTES - 4 * fwords) / 4 / (PROBE_BLOCK / 64) - 64;
+    const uint32_t per_wave = (LDS_PER_CU - 4 * fwords) / 4 / (PROBE_BLOCK / 64) - 64;
     return per_wave < PROBE_LIST_MAX ? per_wave : PROBE_LIST_MAX;
 }
 static_assert(probe_list_cap(PROBE_FILTER_WORDS) >= PROBE_LIST_MIN, "LDS of the largest filter and the lists");
@@ -667,7 +739,10 @@ __global__ void __launch_bounds__(PROBE_BLOCK) k_probe_full_lds(const int32_t *_
         }
     }
     __syncthreads();
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63;
+    // scalar addresses save the filter's form 11 spilled registers (719 -> 705
+    // us); the value table's form spills none and ran slower with them (233 -> 250)
+    const int wave = VALS ? (int)(threadIdx.x >> 6) : wave_index();
     // the wave's row masks and list, behind the filter
     uint32_t *const hit_of = reinterpret_cast<uint32_t *>(probe_lds) + fwords + wave * (64 + cap);
     uint32_t *const list = hit_of + 64;
@@ -1751,11 +1826,29 @@ void launch_build_keyvals(const int32_t *keys, const int32_t *vals, const uint8_
     check_launch("build_keyvals");
 }
 
+// A semi probe reads a bitmap in LDS where two blocks' bitmaps fit a CU and
+// the column has 128 rows or more per table slot: every block reads the whole
+// table first (16M rows, 300,000 slots: 21 us without, 26 with; 60M rows 78
+// and 66; 6M rows, 20,000 slots 13 and 11).  A larger table would leave one
+// block per CU (1.4M slots, 200M rows, 4 % flagged: 284 us without, 306 with).
+constexpr int64_t SEMI_LDS_MIN_ROWS = 4 << 20;
+constexpr int64_t SEMI_LDS_MIN_RATIO = 128;
+constexpr int64_t SEMI_LDS_MAX_SLOTS = (int64_t)LDS_PER_CU / 2 * 8;
+
 void launch_probe_semi(const int32_t *probe, const uint8_t *in, uint8_t *out, int64_t n, const uint8_t *ht,
                        int32_t min, int32_t max, hipStream_t s)
 {
     if (n <= 0) return;
     const int vec = aligned(probe, 16) && aligned(in, 4) && aligned(out, 4);
+    const int64_t len = max >= min ? (int64_t)max - min + 1 : 0;
+    if (vec && aligned(ht, 16) && n >= SEMI_LDS_MIN_ROWS && len > 0 && len <= SEMI_LDS_MAX_SLOTS &&
+        len * SEMI_LDS_MIN_RATIO <= n) {
+        const size_t lds = ((size_t)len + 127) / 128 * 16;
+        const dim3 grid(stream_grid(n, (int64_t)SEMI_BLOCK * UNROLL * 4, 2));
+        hipLaunchKernelGGL(k_probe_semi_lds, grid, dim3(SEMI_BLOCK), lds, s, probe, in, out, n, ht, (uint32_t)len, min);
+        check_launch("probe_semi");
+        return;
+    }
     hipLaunchKernelGGL(k_probe_semi, dim3(vec ? grid_rows(n) : grid_one(n)), dim3(BLOCK), 0, s, probe, in, out, n,
                        ht, min, max, vec);
     check_launch("probe_semi");
@@ -1844,8 +1937,6 @@ void launch_count_flags(const uint8_t *flags, int64_t n, uint64_t *out, bool acc
 // LDS budget of the privatised group-by (bytes); the slot array is u64 plus a
 // one-bit occupancy map.
 constexpr uint64_t GROUPBY_LDS_BYTES = 64 * 1024;
-// LDS of one CU (gfx950)
-constexpr size_t GROUPBY_LDS_PER_CU = 160 * 1024;
 
 uint64_t groupby_lds_max_slots() { return (GROUPBY_LDS_BYTES * 8) / (64 + 1); }
 
@@ -1880,7 +1971,7 @@ void launch_groupby_dense(const int32_t *const *keys, int k, const int32_t *mins
         // as many blocks per CU as that LDS allows (at most 2)
         const size_t bytes = prod * 8 + ((prod + 31) / 32) * 4;
         const size_t used = bytes + (GB_BLOCK / 64) * GB_LIST * sizeof(uint16_t);
-        const int per_cu = std::max(1, std::min(2, (int)(GROUPBY_LDS_PER_CU / used)));
+        const int per_cu = std::max(1, std::min(2, (int)(LDS_PER_CU / used)));
         const dim3 grid(stream_grid(n, WT_ROWS * (GB_BLOCK / 64), per_cu));
 #define SDB_GROUPBY_CASE(KV)                                                                                       \
     if (aligned(flags, 4))                                                                                         \

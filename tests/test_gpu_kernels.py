@@ -152,3 +152,28 @@ def test_probe_full_folded_filter(ops, length, match):
     s = torch.where(inside, s, 0).long()
     hit = (fl != 0) & inside & (pairs[0::2][s] == 1)
     assert bool((out == hit).all()) and bool((vo == torch.where(hit, pairs[1::2][s], -7)).all())
+
+
+# Semi probes over at least 4M rows and 128 rows per table slot read a bitmap
+# in LDS: one slot, around the 16 slots a thread packs, a table that is not
+# 16-byte aligned (no bitmap), the largest table and one slot more; in place.
+@pytest.mark.parametrize("length,off,flagged", [
+    (1, 0, 1.0), (15, 0, 0.5), (17, 0, 1.0), (61_130, 0, 0.02), (61_130, 1, 1.0), (300_000, 0, 0.9),
+    (655_360, 0, 0.9), (655_361, 0, 0.9)])
+def test_probe_semi_lds_tables(ops, length, off, flagged):
+    import torch
+    g = torch.Generator("cuda").manual_seed(length)
+    n, mn = max(128 * length, 4 << 20) + 3, -1000
+    ht = torch.zeros(length + off, dtype=torch.uint8, device="cuda")
+    ht[off:] = torch.randint(0, 3, (length,), generator=g, device="cuda", dtype=torch.uint8) * 127
+    ht = ht[off:]
+    probe = torch.randint(mn - length // 8 - 1, mn + length + length // 8 + 1, (n,), generator=g, device="cuda",
+                          dtype=torch.int32)
+    probe[:3] = torch.tensor([-2**31, 2**31 - 1, mn + length - 1], dtype=torch.int32, device="cuda")
+    fl = (torch.rand(n, generator=g, device="cuda") < flagged).to(torch.uint8) * 3
+    s = probe - mn  # the two extreme keys wrap to far outside
+    inside = (s >= 0) & (s < length)
+    want = (fl != 0) & inside & (ht[torch.where(inside, s, 0)] != 0)
+    ops.filter_join(probe, fl, n, ht, mn, mn + length - 1)
+    assert bool((fl == want).all())
+
