@@ -9,7 +9,6 @@
 #include <chrono>
 #include <cstdint>
 #include <deque>
-#include <functional>
 #include <map>
 #include <memory>
 #include <string>
@@ -289,8 +288,7 @@ struct NotBatchable : std::runtime_error {
 // (sdb_engine_execute_batch): while active, the fused program of every
 // bundle over `table` is recorded instead of launched, the table's row-sized
 // intermediates get placeholder addresses (never registered, so a launch
-// that would touch one fails its bounds check), and device work that must
-// follow the fact pass is deferred.
+// that would touch one fails its bounds check).
 struct CapturedBundle {
     FProgram p;
     int64_t n;
@@ -311,7 +309,6 @@ struct Capture {
     std::string table;
     uint32_t lds_budget = F_LDS_BUDGET;           // LDS one captured program may use
     std::vector<CapturedBundle> bundles;
-    std::vector<std::function<void()>> deferred;  // run after the batched fact pass
     uint64_t phantom_next = 0;
 };
 
@@ -416,8 +413,9 @@ class TransientTable {
 
     uint64_t get_nrows() const { return nrows_; }
     const std::vector<Column *> &get_columns() const { return current_columns_; }
-    // Device flags of the table (materialised if still all-true).
-    const uint8_t *flags_device();
+    // The table's selection: its flags, or what stands for them while they
+    // have not been written (as FinalTable).
+    void selection(const uint8_t *&flags, const uint32_t *&seen) const;
 
   private:
     // throws unless the flags buffer is registered device memory (a captured
@@ -439,6 +437,9 @@ class TransientTable {
     uint8_t *flags_ = nullptr, *flags_secondary_ = nullptr;
     uint8_t *virgin_ = nullptr;          // flags buffer that is logically all
                                          // true and not yet written
+    const uint32_t *seen_ = nullptr;     // the group-by's occupied slots, while
+                                         // flags_ is not yet written from them
+    void write_seen_flags();
     // estimated fraction of rows the filters so far keep (from the column
     // statistics; it orders fused predicates, never decides a result)
     float est_kept_ = 1.0f;
@@ -494,7 +495,10 @@ struct ResultTable {
 // The final table of a plan, on the device (valid until the allocator resets).
 struct FinalTable {
     uint64_t nrows = 0;
+    // Its selection: the flags; else the group-by's `seen` words; else every
+    // row is selected.
     const uint8_t *flags = nullptr;
+    const uint32_t *seen = nullptr;
     struct Col {
         const void *data;
         bool is_u64;

@@ -392,7 +392,6 @@ std::vector<ResultTable> execute_batch(Engine &eng, const std::vector<PlanResult
     struct Pipe {
         FinalTable fin;
         std::vector<CapturedBundle> bundles;
-        std::vector<std::function<void()>> deferred;
         bool batched = false;
     };
     std::vector<Pipe> pipes(n);
@@ -412,7 +411,6 @@ std::vector<ResultTable> execute_batch(Engine &eng, const std::vector<PlanResult
             if (ok) {
                 pipes[i].fin = fin;
                 pipes[i].bundles = std::move(eng.capture.bundles);
-                pipes[i].deferred = std::move(eng.capture.deferred);
                 pipes[i].batched = true;
             } else if (debug_batch()) {
                 fprintf(stderr, "[batch] plan %d runs alone: %zu captured bundles\n", i, eng.capture.bundles.size());
@@ -483,8 +481,6 @@ std::vector<ResultTable> execute_batch(Engine &eng, const std::vector<PlanResult
             for (int i : members) pipes[i].batched = false;
             members.clear();
         }
-        for (int i : members)
-            for (auto &f : pipes[i].deferred) f();
     }
     const double t_shared = ms_since(t0);
     for (int i = 0; i < n; i++)

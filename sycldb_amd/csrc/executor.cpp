@@ -214,7 +214,7 @@ FinalTable run_ddor_plan(Engine &eng, const PlanResult &plan)
 
     FinalTable t;
     t.nrows = final_table.get_nrows();
-    t.flags = final_table.flags_device();
+    final_table.selection(t.flags, t.seen);
     for (Column *c : final_table.get_columns()) {
         if (!c || !c->loaded || !c->data) continue;
         t.cols.push_back({c->data, c->is_aggregate, std::min(t.nrows, c->nrows)});
@@ -270,7 +270,7 @@ constexpr uint64_t RESULT_SPARSE_MIN_ROWS = 1u << 15;
 
 bool sparse_result(const FinalTable &t)
 {
-    if (t.nrows < RESULT_SPARSE_MIN_ROWS || t.nrows >= (1ull << 31) || !t.flags ||
+    if (t.nrows < RESULT_SPARSE_MIN_ROWS || t.nrows >= (1ull << 31) || (!t.flags && !t.seen) ||
         t.cols.size() > (size_t)GATHER_MAX_COLS)
         return false;
     for (const FinalTable::Col &c : t.cols)
@@ -280,87 +280,141 @@ bool sparse_result(const FinalTable &t)
 
 // Device-to-host copies through the engine's pinned staging buffer: every
 // copy queued, one wait for the stream, then into host memory.  Up to
-// PACK_MAX_BYTES in all, the arrays are first packed on the device.
+// PACK_DIRECT_BYTES in all, one kernel writes the arrays straight into the
+// staging buffer; up to PACK_MAX_BYTES they are packed on the device first and
+// cross PCIe in one transfer.  (A q2.x result, 119 KB in four arrays: packing,
+// transfer and the gap between them 8 us, the direct writes 4.)
+constexpr size_t PACK_DIRECT_BYTES = size_t(1) << 20;
 constexpr size_t PACK_MAX_BYTES = size_t(64) << 20;
 struct HostCopies {
     struct Part {
         const void *src;
         void *dst;
         size_t off, bytes;
+        PackKind kind;
     };
     std::vector<Part> parts;
     size_t total = 0;
-    void add(const void *src, void *dst, size_t bytes)
+    void add(const void *src, void *dst, size_t bytes, PackKind kind = PACK_COPY)
     {
         if (!bytes) return;
         total = (total + 15) / 16 * 16;
-        parts.push_back({src, dst, total, bytes});
+        parts.push_back({src, dst, total, bytes, kind});
         total += bytes;
     }
-    void run(Engine &eng)
+    void pack(Engine &eng, uint8_t *to)
     {
-        if (parts.empty()) {
-            eng.wait_stream();
+        PackParts pk{};
+        for (size_t i = 0; i < parts.size(); i++) {
+            pk.src[pk.n] = static_cast<const uint8_t *>(parts[i].src);
+            pk.off[pk.n] = parts[i].off;
+            pk.bytes[pk.n] = parts[i].bytes;
+            pk.kind[pk.n] = parts[i].kind;
+            if (++pk.n == PACK_MAX_PARTS || i + 1 == parts.size()) {
+                launch_pack_parts(pk, to, eng.stream);
+                eng.launches++;
+                pk.n = 0;
+            }
+        }
+    }
+    // queues the copies into `host` (total bytes of pinned memory)
+    void queue(Engine &eng, uint8_t *host)
+    {
+        if (total <= PACK_DIRECT_BYTES) {
+            pack(eng, host);
             return;
         }
-        uint8_t *host = static_cast<uint8_t *>(eng.pinned_buffer(total));
-        if (parts.size() == 1 || total > PACK_MAX_BYTES) {
-            for (const Part &p : parts)
-                SDB_HIP(hipMemcpyAsync(host + p.off, p.src, p.bytes, hipMemcpyDeviceToHost, eng.stream));
-        } else {
-            // several arrays: packed on the device into the staging layout,
-            // then one transfer (each transfer costs ~10 us of latency)
+        if (total <= PACK_MAX_BYTES) {
             uint8_t *dev = eng.mm->alloc<uint8_t>(total);
-            PackParts pk{};
-            for (const Part &p : parts) {
-                pk.src[pk.n] = static_cast<const uint8_t *>(p.src);
-                pk.off[pk.n] = p.off;
-                pk.bytes[pk.n] = p.bytes;
-                if (++pk.n == PACK_MAX_PARTS) {
-                    launch_pack_parts(pk, dev, eng.stream);
-                    eng.launches++;
-                    pk.n = 0;
-                }
-            }
-            if (pk.n) {
-                launch_pack_parts(pk, dev, eng.stream);
-                eng.launches++;
-            }
+            pack(eng, dev);
             SDB_HIP(hipMemcpyAsync(host, dev, total, hipMemcpyDeviceToHost, eng.stream));
+            return;
         }
+        for (const Part &p : parts) {
+            if (p.kind == PACK_TRUE) {
+                std::memset(host + p.off, 1, p.bytes);
+                continue;
+            }
+            const void *src = p.src;
+            if (p.kind == PACK_SEEN) {
+                uint8_t *flags = eng.mm->alloc<uint8_t>(p.bytes);
+                launch_seen_to_flags(static_cast<const uint32_t *>(p.src), flags, p.bytes, eng.stream);
+                eng.launches++;
+                src = flags;
+            }
+            SDB_HIP(hipMemcpyAsync(host + p.off, src, p.bytes, hipMemcpyDeviceToHost, eng.stream));
+        }
+    }
+    void wait(Engine &eng)
+    {
         eng.mark("result wait");
         eng.wait_stream();
         eng.mark("result ready");
+    }
+    // after the wait
+    void deliver(const uint8_t *host)
+    {
         for (const Part &p : parts) std::memcpy(p.dst, host + p.off, p.bytes);
         parts.clear();
         total = 0;
     }
 };
 
+// Sparse tables whose largest possible result fits the staging buffer
+// (SPARSE_STAGE_MAX for all of a call's) have their selected rows written
+// there by the kernels that find them.
+constexpr size_t SPARSE_STAGE_MAX = size_t(64) << 20;
+
+size_t sparse_stage_bytes(const FinalTable &t)
+{
+    size_t b = 16 + (t.nrows * 4 + 15) / 16 * 16; // count, row ids
+    for (const FinalTable::Col &c : t.cols) b += (t.nrows * (c.is_u64 ? 8 : 4) + 15) / 16 * 16;
+    return b;
+}
+
 } // namespace
 
 std::vector<ResultTable> copy_results(Engine &eng, const std::vector<FinalTable> &ts)
 {
     // host copies of the final tables (the materialize_host_view +
-    // save_result path, executor/result_writer.cpp:28-67), all tables in
-    // at most two waits for the stream
+    // save_result path, executor/result_writer.cpp:28-67), all tables in one
+    // wait for the stream (two when a large group-by does not fit the staging)
     std::vector<ResultTable> out(ts.size());
     HostCopies copies;
-    std::vector<size_t> sparse;
-    for (size_t i = 0; i < ts.size(); i++)
-        if (sparse_result(ts[i])) sparse.push_back(i);
-    // large group-by tables: the selected row ids, compacted in row order on
-    // the device; their counts come back with the dense tables
+    std::vector<size_t> sparse, staged; // staged: written into the staging buffer by the device
+    size_t stage_total = 0;
+    for (size_t i = 0; i < ts.size(); i++) {
+        const FinalTable &t = ts[i];
+        if (!sparse_result(t)) continue;
+        out[i].sparse = true;
+        const size_t b = sparse_stage_bytes(t);
+        if (t.nrows <= SPARSE_MAX_ROWS && stage_total + b <= SPARSE_STAGE_MAX) {
+            staged.push_back(i);
+            stage_total += b;
+        } else {
+            sparse.push_back(i);
+        }
+    }
+    // the other large group-by tables: the selected row ids, compacted in row
+    // order on the device; their counts come back with the dense tables
     std::vector<int32_t *> ids(ts.size(), nullptr);
     std::vector<uint32_t> counts(sparse.size(), 0);
     if (!sparse.empty()) {
         uint32_t *d_counts = eng.mm->alloc<uint32_t>(sparse.size());
         for (size_t j = 0; j < sparse.size(); j++) {
             const FinalTable &t = ts[sparse[j]];
-            eng.registry.check(t.flags, t.nrows, "result flags");
+            const uint8_t *flags = t.flags;
+            if (!flags) {
+                eng.registry.check(t.seen, t.nrows * 4, "result group-by slots");
+                uint8_t *f = eng.mm->alloc<uint8_t>(t.nrows);
+                launch_seen_to_flags(t.seen, f, t.nrows, eng.stream);
+                eng.launches++;
+                flags = f;
+            }
+            eng.registry.check(flags, t.nrows, "result flags");
             int32_t *row_ids = eng.mm->alloc<int32_t>(t.nrows);
             uint32_t *tiles = eng.mm->alloc<uint32_t>((uint64_t)std::max<int64_t>(compact_tiles((int64_t)t.nrows), 1));
-            launch_compact_into(t.flags, (int64_t)t.nrows, row_ids, d_counts + j, tiles, eng.stream);
+            launch_compact_into(flags, (int64_t)t.nrows, row_ids, d_counts + j, tiles, eng.stream);
             eng.launches += 3;
             ids[sparse[j]] = row_ids;
         }
@@ -370,7 +424,6 @@ std::vector<ResultTable> copy_results(Engine &eng, const std::vector<FinalTable>
         const FinalTable &t = ts[i];
         ResultTable &res = out[i];
         res.nrows = t.nrows;
-        res.sparse = ids[i] != nullptr;
         for (const FinalTable::Col &c : t.cols) {
             ResultTable::Col rc;
             rc.is_u64 = c.is_u64;
@@ -379,8 +432,10 @@ std::vector<ResultTable> copy_results(Engine &eng, const std::vector<FinalTable>
         if (res.sparse) continue;
         res.flags.resize(res.nrows);
         if (res.nrows) {
-            eng.registry.check(t.flags, res.nrows, "result flags");
-            copies.add(t.flags, res.flags.data(), res.nrows);
+            if (t.flags) eng.registry.check(t.flags, res.nrows, "result flags");
+            else if (t.seen) eng.registry.check(t.seen, res.nrows * 4, "result group-by slots");
+            copies.add(t.flags ? (const void *)t.flags : (const void *)t.seen, res.flags.data(), res.nrows,
+                       t.flags ? PACK_COPY : t.seen ? PACK_SEEN : PACK_TRUE);
         }
         for (size_t c = 0; c < t.cols.size(); c++) {
             const FinalTable::Col &fc = t.cols[c];
@@ -394,10 +449,57 @@ std::vector<ResultTable> copy_results(Engine &eng, const std::vector<FinalTable>
             }
         }
     }
-    copies.run(eng);
-    // large group-by tables: every column gathered at the selected rows on
-    // the device, then copied
-    bool any = false;
+    // one staging buffer: the packed arrays, then the staged sparse tables
+    const size_t stage_off = (copies.total + 15) / 16 * 16;
+    uint8_t *host = static_cast<uint8_t *>(eng.pinned_buffer(std::max<size_t>(stage_off + stage_total, 1)));
+    std::vector<SparseTable> st(staged.size());
+    uint8_t *at = host + stage_off;
+    auto take = [&at](size_t bytes) {
+        uint8_t *p = at;
+        at += (bytes + 15) / 16 * 16;
+        return p;
+    };
+    for (size_t j = 0; j < staged.size(); j++) {
+        const FinalTable &t = ts[staged[j]];
+        SparseTable &s = st[j];
+        s = SparseTable{};
+        if (t.flags) eng.registry.check(t.flags, t.nrows, "result flags");
+        else eng.registry.check(t.seen, t.nrows * 4, "result group-by slots");
+        s.flags = t.flags;
+        s.seen = t.seen;
+        s.rows = (uint32_t)t.nrows;
+        s.counts = eng.mm->alloc<uint32_t>(sparse_tiles(t.nrows));
+        s.count = reinterpret_cast<uint32_t *>(take(4));
+        s.ids = reinterpret_cast<uint32_t *>(take(t.nrows * 4));
+        s.ncols = (int32_t)t.cols.size();
+        for (size_t c = 0; c < t.cols.size(); c++) {
+            const FinalTable::Col &fc = t.cols[c];
+            const uint64_t elem = fc.is_u64 ? 8 : 4;
+            if (fc.rows) eng.registry.check(fc.data, fc.rows * elem, "result column");
+            s.src[c] = fc.data;
+            s.src_rows[c] = (uint32_t)std::min<uint64_t>(fc.rows, t.nrows);
+            if (fc.is_u64) s.is_u64 |= 1u << c;
+            s.dst[c] = take(t.nrows * elem);
+        }
+    }
+    if (!copies.parts.empty()) copies.queue(eng, host);
+    if (!st.empty()) eng.launches += launch_sparse_tables(st.data(), st.size(), eng.stream);
+    copies.wait(eng);
+    copies.deliver(host);
+    for (size_t j = 0; j < staged.size(); j++) {
+        ResultTable &res = out[staged[j]];
+        const SparseTable &s = st[j];
+        const uint32_t k = *s.count;
+        if (k > s.rows) fail(SDB_ERR_RUNTIME, "result compaction: selected count out of range");
+        res.sel.assign(s.ids, s.ids + k);
+        for (size_t c = 0; c < res.cols.size(); c++) {
+            ResultTable::Col &rc = res.cols[c];
+            if (rc.is_u64) rc.u64.assign(static_cast<const uint64_t *>(s.dst[c]), static_cast<const uint64_t *>(s.dst[c]) + k);
+            else rc.i32.assign(static_cast<const int32_t *>(s.dst[c]), static_cast<const int32_t *>(s.dst[c]) + k);
+        }
+    }
+    // the large ones that were not staged: every column gathered at the
+    // selected rows on the device, then copied
     for (size_t j = 0; j < sparse.size(); j++) {
         const FinalTable &t = ts[sparse[j]];
         ResultTable &res = out[sparse[j]];
@@ -405,7 +507,6 @@ std::vector<ResultTable> copy_results(Engine &eng, const std::vector<FinalTable>
         if (k > t.nrows) fail(SDB_ERR_RUNTIME, "result compaction: selected count out of range");
         res.sel.resize(k);
         if (!k) continue;
-        any = true;
         GatherCols g{};
         g.ncols = (int32_t)t.cols.size();
         for (size_t c = 0; c < t.cols.size(); c++) {
@@ -426,7 +527,12 @@ std::vector<ResultTable> copy_results(Engine &eng, const std::vector<FinalTable>
         eng.launches++;
         copies.add(ids[sparse[j]], res.sel.data(), (size_t)k * 4);
     }
-    if (any) copies.run(eng);
+    if (!copies.parts.empty()) {
+        host = static_cast<uint8_t *>(eng.pinned_buffer(copies.total));
+        copies.queue(eng, host);
+        copies.wait(eng);
+        copies.deliver(host);
+    }
     return out;
 }
 

@@ -1586,21 +1586,143 @@ __global__ void __launch_bounds__(BLOCK) k_gather_cols(GatherCols g, const int32
 }
 
 // blockIdx.y = part; the blocks of a part stride over its bytes (16 at a
-// time where source and destination allow, the rest one by one)
-__global__ void __launch_bounds__(BLOCK) k_pack_parts(PackParts p, uint8_t *dst)
+// time where source and destination allow, the rest one by one).  One
+// result's few parts come as a short argument list.
+constexpr int PACK_FEW = 8;
+template <int N> struct PackList {
+    const uint8_t *src[N];
+    uint64_t off[N];
+    uint64_t bytes[N];
+    uint8_t kind[N];
+};
+
+template <int N> __global__ void __launch_bounds__(BLOCK) k_pack_parts(PackList<N> p, uint8_t *dst)
 {
     const int i = blockIdx.y;
     const uint8_t *src = p.src[i];
+    const uint32_t *seen = reinterpret_cast<const uint32_t *>(src);
     uint8_t *out = dst + p.off[i];
     const uint64_t bytes = p.bytes[i];
+    const uint32_t kind = p.kind[i];
     const uint64_t stride = (uint64_t)gridDim.x * BLOCK;
     uint64_t head = 0;
     if ((((uintptr_t)src | (uintptr_t)out) & 15) == 0) {
         head = bytes & ~uint64_t(15);
-        for (uint64_t j = (uint64_t)blockIdx.x * BLOCK + threadIdx.x; j < head / 16; j += stride)
-            reinterpret_cast<uint4 *>(out)[j] = reinterpret_cast<const uint4 *>(src)[j];
+        for (uint64_t j = (uint64_t)blockIdx.x * BLOCK + threadIdx.x; j < head / 16; j += stride) {
+            uint4 q = make_uint4(0x01010101u, 0x01010101u, 0x01010101u, 0x01010101u);
+            if (kind == PACK_COPY) q = reinterpret_cast<const uint4 *>(src)[j];
+            else if (kind == PACK_SEEN) {
+                uint32_t w[4];
+#pragma unroll
+                for (int k = 0; k < 4; k++) {
+                    const uint4 x = reinterpret_cast<const uint4 *>(seen)[4 * j + k];
+                    w[k] = (uint32_t)(x.x != 0) | (uint32_t)(x.y != 0) << 8 | (uint32_t)(x.z != 0) << 16 |
+                           (uint32_t)(x.w != 0) << 24;
+                }
+                q = make_uint4(w[0], w[1], w[2], w[3]);
+            }
+            reinterpret_cast<uint4 *>(out)[j] = q;
+        }
     }
-    for (uint64_t j = head + (uint64_t)blockIdx.x * BLOCK + threadIdx.x; j < bytes; j += stride) out[j] = src[j];
+    for (uint64_t j = head + (uint64_t)blockIdx.x * BLOCK + threadIdx.x; j < bytes; j += stride)
+        out[j] = kind == PACK_COPY ? src[j] : kind == PACK_SEEN ? (uint8_t)(seen[j] != 0) : (uint8_t)1;
+}
+
+// Selected rows of sparse result tables.  The rows cross PCIe where they are
+// found: the host needs no count first, so it waits once and no gather,
+// packing or transfer follows (the results of a 437,500-slot group-by took
+// nine launches and two waits).  A tile is 2,048 rows, 8 per thread; the
+// write pass adds up the tiles' counts before its own.
+constexpr int SPARSE_TABLES = 8; // per launch
+constexpr uint32_t SPARSE_TILE = 8 * BLOCK;
+struct SparseJobs {
+    uint32_t first[SPARSE_TABLES]; // first block of each table (unused: UINT32_MAX)
+    SparseTable t[SPARSE_TABLES];
+};
+static_assert(sizeof(SparseJobs) <= 4096, "kernel argument segment");
+
+__device__ __forceinline__ int sparse_job(const SparseJobs &jobs)
+{
+    int j = 0;
+#pragma unroll
+    for (int k = 1; k < SPARSE_TABLES; k++) j += blockIdx.x >= jobs.first[k];
+    return j;
+}
+
+// bit k: row r + k is selected (r: a multiple of 8)
+__device__ __forceinline__ uint32_t sparse_mask(const SparseTable &t, uint32_t r)
+{
+    uint32_t m = 0;
+    if (r + 8u <= t.rows) {
+        if (t.flags) {
+            const uint2 f = *reinterpret_cast<const uint2 *>(t.flags + r);
+            return nz_mask(f.x) | nz_mask(f.y) << 4;
+        }
+        const uint4 a = *reinterpret_cast<const uint4 *>(t.seen + r), b = *reinterpret_cast<const uint4 *>(t.seen + r + 4);
+        return (uint32_t)(a.x != 0) | (uint32_t)(a.y != 0) << 1 | (uint32_t)(a.z != 0) << 2 | (uint32_t)(a.w != 0) << 3 |
+               (uint32_t)(b.x != 0) << 4 | (uint32_t)(b.y != 0) << 5 | (uint32_t)(b.z != 0) << 6 | (uint32_t)(b.w != 0) << 7;
+    }
+    for (uint32_t k = 0; r + k < t.rows; k++) m |= (uint32_t)(t.flags ? t.flags[r + k] != 0 : t.seen[r + k] != 0) << k;
+    return m;
+}
+
+// Sum over the block (valid in every thread); `part` is BLOCK / 64 words of LDS
+__device__ __forceinline__ uint32_t block_sum(uint32_t v, uint32_t *part)
+{
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+    __syncthreads();
+    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = v;
+    __syncthreads();
+    uint32_t s = 0;
+#pragma unroll
+    for (int w = 0; w < BLOCK / 64; w++) s += part[w];
+    return s;
+}
+
+__global__ void __launch_bounds__(BLOCK) k_sparse_count(SparseJobs jobs)
+{
+    __shared__ uint32_t part[BLOCK / 64];
+    const int j = sparse_job(jobs);
+    const uint32_t tile = blockIdx.x - jobs.first[j];
+    const uint32_t c = block_sum(__popc(sparse_mask(jobs.t[j], tile * SPARSE_TILE + 8u * threadIdx.x)), part);
+    if (threadIdx.x == 0) jobs.t[j].counts[tile] = c;
+}
+
+__global__ void __launch_bounds__(BLOCK) k_sparse_write(SparseJobs jobs)
+{
+    __shared__ uint32_t part[BLOCK / 64], wave_count[BLOCK / 64];
+    __shared__ uint16_t list[SPARSE_TILE];
+    const int j = sparse_job(jobs);
+    const SparseTable &t = jobs.t[j];
+    const uint32_t tile = blockIdx.x - jobs.first[j], t0 = tile * SPARSE_TILE;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    uint32_t m = sparse_mask(t, t0 + 8u * threadIdx.x), before = 0;
+    for (uint32_t i = threadIdx.x; i < tile; i += BLOCK) before += t.counts[i];
+    const uint32_t base = block_sum(before, part);
+    uint32_t total;
+    uint32_t at = wave_prefix((uint32_t)__popc(m), lane, total);
+    if (lane == 0) wave_count[wave] = total;
+    __syncthreads();
+    uint32_t count = 0;
+#pragma unroll
+    for (int w = 0; w < BLOCK / 64; w++) {
+        if (w < wave) at += wave_count[w];
+        count += wave_count[w];
+    }
+    for (; m; m &= m - 1) list[at++] = (uint16_t)(8u * threadIdx.x + (uint32_t)__builtin_ctz(m));
+    __syncthreads();
+    for (uint32_t i = threadIdx.x; i < count; i += BLOCK) t.ids[base + i] = t0 + list[i];
+    for (int c = 0; c < t.ncols; c++) {
+        const bool wide = (t.is_u64 >> c) & 1u;
+        for (uint32_t i = threadIdx.x; i < count; i += BLOCK) {
+            const uint32_t r = t0 + list[i];
+            const bool in = r < t.src_rows[c];
+            if (wide) static_cast<uint64_t *>(t.dst[c])[base + i] = in ? static_cast<const uint64_t *>(t.src[c])[r] : 0ull;
+            else static_cast<int32_t *>(t.dst[c])[base + i] = in ? static_cast<const int32_t *>(t.src[c])[r] : 0;
+        }
+    }
+    if (threadIdx.x == 0 && t0 + SPARSE_TILE >= t.rows) *t.count = base + count;
 }
 
 // The statistics of compact probe tables (one block per table): the sum of
@@ -2148,8 +2270,46 @@ void launch_pack_parts(const PackParts &p, uint8_t *dst, hipStream_t s)
     uint64_t most = 0;
     for (int i = 0; i < p.n; i++) most = std::max(most, p.bytes[i]);
     const unsigned gx = (unsigned)std::max<uint64_t>(1, std::min<uint64_t>((most / 16 + BLOCK - 1) / BLOCK, 256));
-    hipLaunchKernelGGL(k_pack_parts, dim3(gx, (unsigned)p.n), dim3(BLOCK), 0, s, p, dst);
+    auto launch = [&](auto list) {
+        for (int i = 0; i < p.n; i++) {
+            list.src[i] = p.src[i];
+            list.off[i] = p.off[i];
+            list.bytes[i] = p.bytes[i];
+            list.kind[i] = p.kind[i];
+        }
+        constexpr int N = sizeof(list.kind);
+        hipLaunchKernelGGL((k_pack_parts<N>), dim3(gx, (unsigned)p.n), dim3(BLOCK), 0, s, list, dst);
+    };
+    if (p.n <= PACK_FEW) launch(PackList<PACK_FEW>{});
+    else launch(PackList<PACK_MAX_PARTS>{});
     check_launch("pack_parts");
+}
+
+uint64_t sparse_tiles(uint64_t rows) { return (rows + SPARSE_TILE - 1) / SPARSE_TILE; }
+
+int launch_sparse_tables(const SparseTable *t, size_t n, hipStream_t s)
+{
+    int launches = 0;
+    for (size_t at = 0; at < n; at += SPARSE_TABLES) {
+        SparseJobs jobs{};
+        std::fill(std::begin(jobs.first), std::end(jobs.first), UINT32_MAX);
+        uint32_t blocks = 0;
+        for (size_t i = 0; i < (size_t)SPARSE_TABLES && at + i < n; i++) {
+            const SparseTable &T = t[at + i];
+            if (T.rows == 0 || T.rows > SPARSE_MAX_ROWS || T.ncols > GATHER_MAX_COLS || (!T.flags && !T.seen) ||
+                !aligned(T.flags, 8) || !aligned(T.seen, 16))
+                fail(SDB_ERR_RUNTIME, "sparse result table out of the kernels' range");
+            jobs.first[i] = blocks;
+            jobs.t[i] = T;
+            blocks += (uint32_t)sparse_tiles(T.rows);
+        }
+        if (!blocks) continue;
+        hipLaunchKernelGGL(k_sparse_count, dim3(blocks), dim3(BLOCK), 0, s, jobs);
+        hipLaunchKernelGGL(k_sparse_write, dim3(blocks), dim3(BLOCK), 0, s, jobs);
+        check_launch("sparse_tables");
+        launches += 2;
+    }
+    return launches;
 }
 
 void launch_gather_i32(const int32_t *src, const int32_t *ids, int64_t count, int32_t *dst, hipStream_t s)

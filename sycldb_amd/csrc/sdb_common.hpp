@@ -60,16 +60,42 @@ struct GatherCols {
     int32_t ncols;
 };
 void launch_gather_cols(const GatherCols &g, const int32_t *ids, int64_t count, hipStream_t s);
-// Copies device buffers src[i] (bytes[i] bytes) to dst + off[i]: several
-// small arrays packed into one buffer for a single transfer.
+// Writes bytes[i] bytes to dst + off[i] for every part: several small arrays
+// packed into one buffer, in device memory or in pinned host memory.
+enum PackKind : uint8_t {
+    PACK_COPY = 0, // the bytes at src[i]
+    PACK_SEEN = 1, // flags: 1 where the uint32 at src[i] is nonzero
+    PACK_TRUE = 2  // flags: all 1 (no source)
+};
 constexpr int PACK_MAX_PARTS = 64;
 struct PackParts {
     const uint8_t *src[PACK_MAX_PARTS];
     uint64_t off[PACK_MAX_PARTS];
     uint64_t bytes[PACK_MAX_PARTS];
+    uint8_t kind[PACK_MAX_PARTS];
     int32_t n;
 };
 void launch_pack_parts(const PackParts &p, uint8_t *dst, hipStream_t s);
+
+// The selected rows of tables of up to SPARSE_MAX_ROWS rows, in row order:
+// their ids, their values of every column (as launch_gather_cols) and their
+// number, written to dst / ids / count (pinned host memory).  A row is
+// selected where its flag (or, without flags, its `seen` word) is nonzero.
+// counts: sparse_tiles(rows) words of device memory.
+constexpr uint64_t SPARSE_MAX_ROWS = 1u << 22;
+struct SparseTable {
+    const uint8_t *flags;
+    const uint32_t *seen;
+    uint32_t *counts;
+    const void *src[GATHER_MAX_COLS];
+    void *dst[GATHER_MAX_COLS];
+    uint32_t src_rows[GATHER_MAX_COLS];
+    uint32_t *ids, *count;
+    uint32_t rows, is_u64;
+    int32_t ncols;
+};
+uint64_t sparse_tiles(uint64_t rows);
+int launch_sparse_tables(const SparseTable *t, size_t n, hipStream_t s); // number of launches
 
 // Statistics of compact probe tables, each stats[i] laid out as [overflow
 // flag, nparts[i] partial counts]: the sums and flags go to dst as pairs.

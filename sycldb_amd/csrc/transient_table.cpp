@@ -129,6 +129,7 @@ void TransientTable::swap_flag_buffers()
 
 void TransientTable::add_pending_kernels(std::vector<KernelBundle> ops)
 {
+    write_seen_flags();
     if (pending_kernels_.empty() || pending_kernels_.back().size() != ops.size()) {
         pending_kernels_.push_back(std::move(ops));
         return;
@@ -150,15 +151,22 @@ void TransientTable::check_flags_memory() const
     }
 }
 
-const uint8_t *TransientTable::flags_device()
+void TransientTable::selection(const uint8_t *&flags, const uint32_t *&seen) const
 {
-    if (virgin_ == flags_) {
-        check_flags_memory();
-        launch_fill_u8(flags_, 1, (int64_t)nrows_, eng_.stream);
-        eng_.launches++;
-        virgin_ = nullptr;
-    }
-    return flags_;
+    flags = virgin_ == flags_ || seen_ ? nullptr : flags_;
+    seen = seen_;
+}
+
+// An operator after the group-by reads the flags in memory.
+void TransientTable::write_seen_flags()
+{
+    if (!seen_) return;
+    // a captured plan's fact pass has not run yet
+    if (eng_.capture.active && name_ == eng_.capture.table)
+        throw NotBatchable("an operator follows the fact table's group-by");
+    launch_seen_to_flags(seen_, flags_, nrows_, eng_.stream);
+    eng_.launches++;
+    seen_ = nullptr;
 }
 
 void TransientTable::execute_pending_kernels(bool dead_after)
@@ -492,18 +500,7 @@ void TransientTable::apply_aggregate(const AggType &agg, const std::vector<int64
     execute_pending_kernels(true);
     nrows_ = prod;
     flags_ = eng_.mm->alloc<uint8_t>(prod);
-    if (eng_.capture.active && name_ == eng_.capture.table) {
-        // the fact pass has not run yet: convert after the batched launch
-        uint8_t *f = flags_;
-        Engine *eng = &eng_;
-        eng_.capture.deferred.push_back([=] {
-            launch_seen_to_flags(seen, f, prod, eng->stream);
-            eng->launches++;
-        });
-    } else {
-        launch_seen_to_flags(seen, flags_, prod, eng_.stream);
-        eng_.launches++;
-    }
+    seen_ = seen; // the flags follow from it when an operator needs them
     virgin_ = nullptr;
     flags_secondary_ = nullptr;
     current_columns_.clear();

@@ -1,0 +1,57 @@
+"""The joins' build sides, run several to a launch, and the results' way back,
+at the table sizes where their tiling can go wrong, against the plan oracle."""
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+from oracle import datagen, plan_oracle as PO  # noqa: E402
+from sycldb_amd import plans as PL  # noqa: E402
+from sycldb_amd import schema as S  # noqa: E402
+
+PLANS = [("t1", {"date": ("year", 1992), "disc": (0, 10), "qty": ("lt", 51)}),
+         ("t1", {"date": ("yearmonthnum", 199201), "disc": (1, 3), "qty": ("range", 2, 40)}),
+         ("t1", {"date": ("year_range_and", 1992, 1993), "disc": (4, 6), "qty": ("lt", 25)}),
+         ("t2", {"part": ("category", 1), "s_region": 1}), ("t2", {"part": ("brand_range", 40, 900), "s_region": 2}),
+         ("t3", {"cust": ("region", 1), "supp": ("region", 1), "date": ("year_range", 1992, 1997), "group": "nation"}),
+         ("t3", {"cust": ("city2", 3, 141), "supp": ("region", 0), "date": ("year_range", 1992, 1997), "group": "city"}),
+         ("t3", {"cust": ("nation", 6), "supp": ("nation", 6), "date": ("yearmonthnum", 199202), "group": "city"}),
+         ("t4", {"c_region": 1, "s_region": 1, "mfgr": (0, 1)}), ("t4", {"c_region": 0, "s_region": 2, "mfgr": (2, 4)})]
+
+
+# 1,024 rows per block and step, 4 per thread: one row, fewer than a thread's,
+# around a block's, around two; the batch holds more builds than one launch takes
+@pytest.mark.parametrize("customer,supplier,part,ddate", [
+    (1, 1, 1, 1), (3, 5, 2, 366), (1023, 1024, 1025, 2556), (2049, 4097, 2047, 1025)])
+def test_build_sides_at_block_edges(customer, supplier, part, ddate):
+    from sycldb_amd.engine import Engine
+    sizes = {"customer": customer, "supplier": supplier, "part": part, "ddate": ddate}
+    rows, seed = 20_011, 45
+    tables = datagen.generate_tables(S, rows, seed, sizes)
+    plans = [PL.build(t, **p) for t, p in PLANS]
+    with Engine() as eng:
+        eng.generate(rows, seed, sizes=sizes)
+        want = [PO.execute_plan(p, tables).rows() for p in plans]
+        for plan, w in zip(plans, want):
+            assert eng.execute(plan).rows() == w, plan
+        got, _ = eng.execute_batch(plans * 3)
+        for g, p, w in zip(got, plans * 3, want * 3):
+            assert g.rows() == w, p
+
+
+def test_many_large_results_in_one_batch():
+    """437,500-slot results: the first six are written to the host by the
+    kernels that find their rows, the others (past the staging buffer's
+    share) compacted and gathered, all beside dense results."""
+    from sycldb_amd.engine import Engine
+    rows, seed = 200_003, 45
+    tables = datagen.generate_tables(S, rows, seed)
+    plans = [PL.build("t3", cust=("region", i % 5), supp=("region", (i * 2 + 1) % 5), date=("year_range", 1992, 1997),
+                      group="city") for i in range(8)]
+    plans[3:3] = [PL.build("t1"), PL.build("t2", part=("category", 1), s_region=1)]
+    plans.append(PL.build("t3", cust=("city2", 1, 2), supp=("city2", 3, 4), date=("yearmonthnum", 199712), group="city"))
+    with Engine() as eng:
+        eng.generate(rows, seed)
+        for _ in range(2):
+            got, _ = eng.execute_batch(plans)
+            for g, p in zip(got, plans):
+                assert g.rows() == PO.execute_plan(p, tables).rows(), p
