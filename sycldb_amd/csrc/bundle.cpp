@@ -109,6 +109,19 @@ void KernelBundle::execute(const ExecContext &ctx) const
                     if (st == ctx.virgin_begin && n == ctx.virgin_end - ctx.virgin_begin) stores_whole = true;
                     else stores_part = true;
                 }
+            // a join's build side waits for the others' (profiled bundles and
+            // forced launch forms run by themselves; a table's segments stay
+            // in order, for keys that several of them hold)
+            DimJob job;
+            if (eng.codegen == SDB_CODEGEN_AUTO && !eng.unroll && ctx.whole_table && !stores_part &&
+                !eng.profiles(ctx.table) && dim_job(p, n, job)) {
+                eng.dim_jobs.push_back(job);
+                if (stores_whole) ctx.virgin_filled = true;
+                eng.mark("queued");
+                return;
+            }
+            eng.mark("program built");
+            eng.flush_builds(); // the bundle may read queued tables
             if (stores_part) {
                 eng.registry.check(ctx.virgin_begin, (uint64_t)(ctx.virgin_end - ctx.virgin_begin), "initial flags");
                 launch_fill_u8(const_cast<uint8_t *>(ctx.virgin_begin), 1, ctx.virgin_end - ctx.virgin_begin, ctx.stream);
@@ -123,7 +136,7 @@ void KernelBundle::execute(const ExecContext &ctx) const
             Engine::ProfRec rec;
             const bool timed = eng.profiles(ctx.table);
             if (timed) eng.prof_begin("fused:" + (ctx.table ? *ctx.table : std::string("?")), n, rec);
-            eng.mark("program built");
+            eng.mark("prepared");
             if (jit) run_fused_jit(L, p, n, ctx.stream);
             else launch_fused(p, n, ctx.stream);
             if (timed) eng.prof_end(rec);
@@ -133,6 +146,7 @@ void KernelBundle::execute(const ExecContext &ctx) const
             return;
         }
     }
+    eng.flush_builds();
     execute_unfused(ctx);
 }
 

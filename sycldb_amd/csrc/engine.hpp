@@ -51,16 +51,8 @@ uint64_t groupby_lds_max_slots();
 // Compact probe tables (ops.hip): bitmap from a uint8 key table, bitmap and
 // uint16 value offsets from a key-value pair table; the set bits counted per
 // block into partials[0, bits_partials(len)) (launch_stats_reduce sums
-// them), *bad set when a value does not fit 16 bits.
+// them), *bad set when a value does not fit 16 bits (launch_compact_tables).
 uint32_t bits_partials(int32_t len);
-void launch_bits_from_keys(const uint8_t *ht, int32_t len, uint32_t *bits, uint32_t *partials, hipStream_t s);
-// Rank dictionary (FV_RANK16 layout) of the presence bitmap of `len` slots
-// and their per-slot 16-bit values; `partials` (or null): the per-block
-// counts launch_bits_from_pairs left for the same table.
-void launch_rank_dict(const uint32_t *bits, int32_t len, const uint16_t *vals, const uint32_t *partials,
-                      uint8_t *dict, uint32_t dict_cap, hipStream_t s);
-void launch_bits_from_pairs(const int32_t *ht, int32_t len, uint32_t *bits, uint16_t *vals, int32_t vmin,
-                            uint32_t *partials, uint32_t *bad, hipStream_t s);
 
 // --------------------------------------------------------- allocation map
 
@@ -253,6 +245,7 @@ struct ExecContext {
     // the all-true buffer stays in use after the bundles: it must end up
     // holding values (stored whole by a program, else filled)
     bool virgin_live = false;
+    bool whole_table = false; // the table is one segment
 };
 
 // KernelBundle, models/execution.hpp:500-651: the operators queued for one
@@ -328,6 +321,14 @@ struct Engine {
     std::vector<std::weak_ptr<CompactState>> pending_compact;
     // Reads the statistics of every pending compact table (one stream sync).
     void resolve_compact();
+    // The joins' build sides and their compact tables still to build: queued
+    // while the joins are walked, built together before the first launch that
+    // may read one (flush_builds).
+    std::vector<DimJob> dim_jobs;
+    std::vector<CompactJob> compact_jobs;
+    void flush_builds();
+    // Releases the previous execution's device memory and queued work.
+    void begin_execution();
     std::map<std::string, std::unique_ptr<Table>> tables;
     int64_t launches = 0;
     double last_device_ms = 0, last_wall_ms = 0;

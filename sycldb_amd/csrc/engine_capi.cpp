@@ -299,10 +299,12 @@ int sdb_engine_execute(sdb_engine *e, const char *plan_json, sdb_result **out)
         const PlanResult plan = parse_plan(plan_json);
         eng.mark("parsed");
         // scratch of the previous query is released (runtime/runtime.cpp:331-345)
-        eng.mm->reset(eng.stream);
+        eng.begin_execution();
+        eng.mark("reset");
         eng.launches = 0;
         const auto w0 = std::chrono::steady_clock::now();
         SDB_HIP(hipEventRecord(eng.ev_start, eng.stream));
+        eng.mark("recorded");
         auto r = std::make_unique<sdb_result>();
         eng.stop_at_wait = true;
         eng.stop_recorded = false;
@@ -388,7 +390,7 @@ std::vector<ResultTable> execute_batch(Engine &eng, const std::vector<PlanResult
     using clk = std::chrono::steady_clock;
     const auto t0 = clk::now();
     auto ms_since = [](clk::time_point a) { return std::chrono::duration<double, std::milli>(clk::now() - a).count(); };
-    eng.mm->reset(eng.stream);
+    eng.begin_execution();
     struct Pipe {
         FinalTable fin;
         std::vector<CapturedBundle> bundles;
@@ -447,6 +449,7 @@ std::vector<ResultTable> execute_batch(Engine &eng, const std::vector<PlanResult
         eng.capture = Capture{};
     }
     const double t_capture = ms_since(t0);
+    eng.flush_builds();
     // the shared fact passes
     std::vector<int> members;
     for (int i = 0; i < n; i++)
@@ -553,7 +556,7 @@ int sdb_engine_reset(sdb_engine *e)
     return guarded([&] {
         require(e, "null engine");
         SDB_HIP(hipSetDevice(e->eng.device));
-        e->eng.mm->reset(e->eng.stream);
+        e->eng.begin_execution();
         SDB_HIP(hipStreamSynchronize(e->eng.stream));
     });
 }

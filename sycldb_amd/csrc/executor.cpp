@@ -211,6 +211,7 @@ FinalTable run_ddor_plan(Engine &eng, const PlanResult &plan)
     }
     TransientTable &final_table = input_of((int64_t)plan.rels.size() - 1);
     final_table.execute_pending_kernels(false);
+    if (!eng.capture.active) eng.flush_builds();
 
     FinalTable t;
     t.nrows = final_table.get_nrows();

@@ -105,4 +105,32 @@ int jit_batch_check(const std::string &arch);
 // covering every instruction form for `arch`; returns how many compiled.
 int jit_check(const std::string &arch);
 
+
+// Build sides run several to a launch (dim.hip): a fused program reduced to
+// selections over whole columns and one hash-table build.
+constexpr int DIM_COLS = 4, DIM_INSTRS = 6;
+constexpr int DIM_JOBS = 20; // per launch (their descriptions are kernel arguments)
+constexpr int64_t DIM_MAX_ROWS = int64_t(4) << 20;
+struct DimInstr {
+    uint8_t kind, cmp, logic; // FK_SEL_LIT / _COL / _RANGE / _IN2 or FK_LOGICAL
+    uint8_t fin, fout, floc;
+    uint8_t a, b;             // columns
+    int32_t lit, lit2;
+};
+struct DimJob {
+    const int32_t *col[DIM_COLS];
+    uint8_t *store;           // flag buffer written from register store_reg, or null
+    void *ht;
+    int32_t n, ht_min, ht_len;
+    uint32_t init;            // flag registers that start true (4 bits each)
+    uint8_t ncols, ninstr, store_reg, vec;
+    uint8_t fin, key, val, pairs; // the build
+    DimInstr ins[DIM_INSTRS];
+};
+// The program as a build job (false: it needs its own kernel).  The program's
+// buffers were checked (validate_program).
+bool dim_job(const FProgram &p, int64_t n, DimJob &job);
+// Runs the jobs, DIM_JOBS to a launch; returns the number of launches.
+int launch_dim_builds(const DimJob *jobs, size_t njobs, hipStream_t s);
+
 } // namespace sdb

@@ -1129,10 +1129,10 @@ __global__ void __launch_bounds__(BLOCK) k_seen_to_flags(const uint32_t *seen, u
 // per block and summed when the statistics are read (k_stats_reduce).
 
 // Stores the block's count (the sum of every wave's, held by its lane 0) in
-// partials[blockIdx.x].  One same-address atomic per block instead
+// *count.  One same-address atomic per block instead
 // serialises: 1,368 blocks over the 1.4M-slot part table took 21 us, 7 us
 // with the partial counts.
-__device__ __forceinline__ void block_count_store(uint32_t local, uint32_t *partials)
+__device__ __forceinline__ void block_count_store(uint32_t local, uint32_t *count)
 {
     __shared__ uint32_t wave_sum[BLOCK / 64];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -1142,7 +1142,7 @@ __device__ __forceinline__ void block_count_store(uint32_t local, uint32_t *part
         uint32_t t = 0;
 #pragma unroll
         for (int w = 0; w < BLOCK / 64; w++) t += wave_sum[w];
-        partials[blockIdx.x] = t;
+        *count = t;
     }
 }
 
@@ -1158,14 +1158,42 @@ __device__ __forceinline__ void block_count_store(uint32_t local, uint32_t *part
 constexpr int BITS_GROUPS = 4;
 constexpr unsigned BITS_MAX_BLOCKS = 2048;
 
-__global__ void __launch_bounds__(BLOCK) k_bits_from_keys(const uint8_t *ht, int32_t len, uint32_t *bits,
-                                                          uint32_t *partials)
+// tables per launch (their descriptions are kernel arguments: the small form
+// for one plan's joins, the large one for a batch's)
+constexpr int COMPACT_JOBS_SMALL = 4, COMPACT_JOBS = 32;
+struct BitsJob {
+    const void *ht;
+    uint32_t *bits;
+    uint16_t *vals;
+    uint32_t *partials, *bad;
+    int32_t len, vmin;
+    uint32_t nblocks, pairs;
+};
+template <int N> struct BitsJobs {
+    uint32_t first[N];
+    BitsJob job[N];
+};
+struct RankJob {
+    const uint32_t *bits, *partials;
+    const uint16_t *vals;
+    uint8_t *dict;
+    int32_t len, words;
+    uint32_t cap_vals;
+};
+template <int N> struct RankJobs {
+    uint32_t first[N];
+    RankJob job[N];
+};
+static_assert(sizeof(BitsJobs<COMPACT_JOBS>) <= 4096 && sizeof(RankJobs<COMPACT_JOBS>) <= 4096, "kernel argument segment");
+
+__device__ __forceinline__ void bits_from_keys(const BitsJob &J, uint32_t block, uint32_t nblocks)
 {
-    const int64_t words = ((int64_t)len + 31) / 32;
+    const uint8_t *ht = static_cast<const uint8_t *>(J.ht);
+    const int64_t len = J.len, words = (len + 31) / 32;
     const int lane = threadIdx.x & 63;
-    const int64_t nwaves = ((int64_t)gridDim.x * BLOCK) >> 6;
+    const int64_t nwaves = ((int64_t)nblocks * BLOCK) >> 6;
     uint32_t local = 0;
-    for (int64_t g0 = (((int64_t)blockIdx.x * BLOCK + threadIdx.x) >> 6) * BITS_GROUPS; g0 * 64 < (int64_t)len;
+    for (int64_t g0 = (((int64_t)block * BLOCK + threadIdx.x) >> 6) * BITS_GROUPS; g0 * 64 < len;
          g0 += nwaves * BITS_GROUPS) {
         bool set[BITS_GROUPS];
 #pragma unroll
@@ -1178,25 +1206,25 @@ __global__ void __launch_bounds__(BLOCK) k_bits_from_keys(const uint8_t *ht, int
             const int64_t g = g0 + k;
             const uint64_t m = __ballot(set[k]);
             if (lane == 0 && 2 * g < words) {
-                bits[2 * g] = (uint32_t)m;
-                if (2 * g + 1 < words) bits[2 * g + 1] = (uint32_t)(m >> 32);
+                J.bits[2 * g] = (uint32_t)m;
+                if (2 * g + 1 < words) J.bits[2 * g + 1] = (uint32_t)(m >> 32);
                 local += (uint32_t)__popcll(m);
             }
         }
     }
-    block_count_store(local, partials);
+    block_count_store(local, J.partials + block);
 }
 
-__global__ void __launch_bounds__(BLOCK) k_bits_from_pairs(const int2 *ht, int32_t len, uint32_t *bits,
-                                                           uint16_t *vals, int32_t vmin, uint32_t *partials,
-                                                           uint32_t *bad)
+__device__ __forceinline__ void bits_from_pairs(const BitsJob &J, uint32_t block, uint32_t nblocks)
 {
-    const int64_t words = ((int64_t)len + 31) / 32;
+    const int2 *ht = static_cast<const int2 *>(J.ht);
+    uint16_t *vals = J.vals;
+    const int64_t len = J.len, words = (len + 31) / 32;
     const int lane = threadIdx.x & 63;
-    const int64_t nwaves = ((int64_t)gridDim.x * BLOCK) >> 6;
+    const int64_t nwaves = ((int64_t)nblocks * BLOCK) >> 6;
     uint32_t local = 0;
     bool ok = true;
-    for (int64_t g0 = (((int64_t)blockIdx.x * BLOCK + threadIdx.x) >> 6) * BITS_GROUPS; g0 * 64 < (int64_t)len;
+    for (int64_t g0 = (((int64_t)block * BLOCK + threadIdx.x) >> 6) * BITS_GROUPS; g0 * 64 < len;
          g0 += nwaves * BITS_GROUPS) {
         int2 e[BITS_GROUPS];
 #pragma unroll
@@ -1209,19 +1237,40 @@ __global__ void __launch_bounds__(BLOCK) k_bits_from_pairs(const int2 *ht, int32
             const int64_t g = g0 + k, s = g * 64 + lane;
             const bool set = e[k].x == 1;
             // unset slots hold VALS_UNSET; a set slot's offset must stay below it
-            const uint32_t d = set ? (uint32_t)e[k].y - (uint32_t)vmin : VALS_UNSET;
+            const uint32_t d = set ? (uint32_t)e[k].y - (uint32_t)J.vmin : VALS_UNSET;
             ok &= !set || d < VALS_UNSET;
             if (vals && s < len) vals[s] = (uint16_t)d;
             const uint64_t m = __ballot(set);
             if (lane == 0 && 2 * g < words) {
-                bits[2 * g] = (uint32_t)m;
-                if (2 * g + 1 < words) bits[2 * g + 1] = (uint32_t)(m >> 32);
+                J.bits[2 * g] = (uint32_t)m;
+                if (2 * g + 1 < words) J.bits[2 * g + 1] = (uint32_t)(m >> 32);
                 local += (uint32_t)__popcll(m);
             }
         }
     }
-    block_count_store(local, partials);
-    if (!ok) atomicOr(bad, 1u);
+    block_count_store(local, J.partials + block);
+    if (!ok) atomicOr(J.bad, 1u);
+}
+
+// Several tables in one launch: block b works on the job whose blocks
+// [first[j], first[j + 1]) hold it (unused entries of first: UINT32_MAX).
+// A launch of 3 to 5 us per table, one after another, made up most of a small
+// query's device time.
+template <int N> __device__ __forceinline__ int job_of(const uint32_t (&first)[N], uint32_t block)
+{
+    int j = 0;
+#pragma unroll
+    for (int k = 1; k < N; k++) j += block >= first[k];
+    return j;
+}
+
+template <int N> __global__ void __launch_bounds__(BLOCK) k_compact_bits(BitsJobs<N> jobs)
+{
+    const int j = job_of(jobs.first, blockIdx.x);
+    const BitsJob &J = jobs.job[j];
+    const uint32_t block = blockIdx.x - jobs.first[j];
+    if (J.pairs) bits_from_pairs(J, block, J.nblocks);
+    else bits_from_keys(J, block, J.nblocks);
 }
 
 // The windows of 32 consecutive keys (one bitmap word) of a table of WB-byte
@@ -1269,7 +1318,7 @@ template <uint32_t WB> struct DictWord {
 
 // Rank dictionary of a presence bitmap with per-slot 16-bit values (the
 // layout FV_RANK16 describes in fused_types.hpp), from the per-block counts
-// of k_bits_from_pairs: its block b counted exactly the slots
+// of bits_from_pairs: its block b counted exactly the slots
 // [1024 b, 1024 b + 1024), i.e. the bitmap words [32 b, 32 b + 32).  One wave
 // per such range: its set slots before the range are the partial counts of
 // the blocks before it; lane l < 32 takes word 32 b + l, the wave scans the
@@ -1277,17 +1326,19 @@ template <uint32_t WB> struct DictWord {
 // slots' values (four vector loads issued together).
 constexpr uint32_t RANK_PART_WORDS = 32;
 
-__global__ void __launch_bounds__(64) k_rank_dict_parts(const uint32_t *__restrict__ bits, int32_t words,
-                                                        const uint32_t *__restrict__ partials,
-                                                        const uint16_t *__restrict__ vals, uint32_t len,
-                                                        uint8_t *__restrict__ dict, uint32_t cap_vals)
+template <int N> __global__ void __launch_bounds__(64) k_rank_dicts(RankJobs<N> jobs)
 {
+    const int j = job_of(jobs.first, blockIdx.x);
+    const RankJob &J = jobs.job[j];
+    const uint32_t *bits = J.bits, *partials = J.partials;
+    const int32_t words = J.words;
+    uint8_t *dict = J.dict;
     const int lane = threadIdx.x;
-    const uint32_t b = blockIdx.x;
+    const uint32_t b = blockIdx.x - jobs.first[j];
     const int32_t w = (int32_t)(b * RANK_PART_WORDS) + (lane & 31);
     const uint32_t m = lane < 32 && w < words ? bits[w] : 0u;
     uint32_t before = 0;
-    for (uint32_t j = lane; j < b; j += 64) before += partials[j];
+    for (uint32_t i = lane; i < b; i += 64) before += partials[i];
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) before += __shfl_xor(before, off, 64);
     const uint32_t c = __popc(m);
@@ -1303,8 +1354,8 @@ __global__ void __launch_bounds__(64) k_rank_dict_parts(const uint32_t *__restri
     reinterpret_cast<uint16_t *>(dict + rank_prefix_off((uint32_t)words))[w] = (uint16_t)base;
     if (m) {
         DictWord<2> x;
-        x.load(reinterpret_cast<const uint8_t *>(vals), len, (uint32_t)w);
-        x.write(m, base, reinterpret_cast<uint16_t *>(dict + rank_values_off((uint32_t)words)), cap_vals);
+        x.load(reinterpret_cast<const uint8_t *>(J.vals), (uint32_t)J.len, (uint32_t)w);
+        x.write(m, base, reinterpret_cast<uint16_t *>(dict + rank_values_off((uint32_t)words)), J.cap_vals);
     }
 }
 
@@ -2132,21 +2183,57 @@ uint32_t bits_partials(int32_t len)
     return (uint32_t)std::min<int64_t>(BITS_MAX_BLOCKS, ((int64_t)len + per_block - 1) / per_block);
 }
 
-void launch_bits_from_keys(const uint8_t *ht, int32_t len, uint32_t *bits, uint32_t *partials, hipStream_t s)
+template <int N> static int launch_tables(const CompactJob *jobs, int n, hipStream_t s)
 {
-    if (len <= 0) return;
-    hipLaunchKernelGGL(k_bits_from_keys, dim3(bits_partials(len)), dim3(BLOCK), 0, s, ht, len, bits, partials);
-    check_launch("bits_from_keys");
+    BitsJobs<N> bj{};
+    RankJobs<N> rj{};
+    std::fill(std::begin(bj.first), std::end(bj.first), UINT32_MAX);
+    std::fill(std::begin(rj.first), std::end(rj.first), UINT32_MAX);
+    uint32_t blocks = 0, ranges = 0;
+    int nbits = 0, nrank = 0;
+    for (int i = 0; i < n; i++) {
+        const CompactJob &c = jobs[i];
+        if (c.len <= 0) continue;
+        if (c.pairs && !aligned(c.ht, 8)) fail(SDB_ERR_INVALID_ARG, "key-value hash table must be 8-byte aligned");
+        const uint32_t nblocks = bits_partials(c.len);
+        bj.first[nbits] = blocks;
+        bj.job[nbits++] = {c.ht, c.bits, c.vals, c.partials, c.bad, c.len, c.vmin, nblocks, c.pairs ? 1u : 0u};
+        blocks += nblocks;
+        if (!c.dict) continue;
+        const uint32_t words = (uint32_t)(((int64_t)c.len + 31) / 32);
+        if (c.dict_cap < rank_values_off(words)) fail(SDB_ERR_RUNTIME, "rank dictionary buffer too small");
+        // the bitmap kernel's blocks each counted one run of 32 words when
+        // the job's blocks cover the table without wrapping (below 2^21
+        // slots; dictionaries are built for tables far smaller)
+        static_assert(64 * BITS_GROUPS * (BLOCK / 64) == 32 * RANK_PART_WORDS, "one bitmap block per 32 words");
+        const uint32_t r = (words + RANK_PART_WORDS - 1) / RANK_PART_WORDS;
+        if (!c.partials || !c.vals || r != nblocks)
+            fail(SDB_ERR_RUNTIME, "rank dictionary: the bitmap's per-block counts do not cover 32 words each");
+        rj.first[nrank] = ranges;
+        rj.job[nrank++] = {c.bits, c.partials, c.vals, c.dict, c.len, (int32_t)words,
+                           (c.dict_cap - rank_values_off(words)) / 2u};
+        ranges += r;
+    }
+    if (nbits) {
+        hipLaunchKernelGGL((k_compact_bits<N>), dim3(blocks), dim3(BLOCK), 0, s, bj);
+        check_launch("compact_bits");
+    }
+    if (nrank) {
+        hipLaunchKernelGGL((k_rank_dicts<N>), dim3(ranges), dim3(64), 0, s, rj);
+        check_launch("rank_dicts");
+    }
+    return (nbits ? 1 : 0) + (nrank ? 1 : 0);
 }
 
-void launch_bits_from_pairs(const int32_t *ht, int32_t len, uint32_t *bits, uint16_t *vals, int32_t vmin,
-                            uint32_t *partials, uint32_t *bad, hipStream_t s)
+int launch_compact_tables(const CompactJob *jobs, size_t njobs, hipStream_t s)
 {
-    if (len <= 0) return;
-    if (!aligned(ht, 8)) fail(SDB_ERR_INVALID_ARG, "key-value hash table must be 8-byte aligned");
-    hipLaunchKernelGGL(k_bits_from_pairs, dim3(bits_partials(len)), dim3(BLOCK), 0, s,
-                       reinterpret_cast<const int2 *>(ht), len, bits, vals, vmin, partials, bad);
-    check_launch("bits_from_pairs");
+    int launches = 0;
+    for (size_t at = 0; at < njobs; at += COMPACT_JOBS) {
+        const int n = (int)std::min<size_t>(COMPACT_JOBS, njobs - at);
+        launches += n <= COMPACT_JOBS_SMALL ? launch_tables<COMPACT_JOBS_SMALL>(jobs + at, n, s)
+                                            : launch_tables<COMPACT_JOBS>(jobs + at, n, s);
+    }
+    return launches;
 }
 
 void launch_stats_reduce(const StatsParts &p, uint32_t *dst, hipStream_t s)
@@ -2155,25 +2242,6 @@ void launch_stats_reduce(const StatsParts &p, uint32_t *dst, hipStream_t s)
     if (p.n > PACK_MAX_PARTS) fail(SDB_ERR_INVALID_ARG, "stats reduce: too many tables");
     hipLaunchKernelGGL(k_stats_reduce, dim3(1, (unsigned)p.n), dim3(BLOCK), 0, s, p, dst);
     check_launch("stats_reduce");
-}
-
-void launch_rank_dict(const uint32_t *bits, int32_t len, const uint16_t *vals, const uint32_t *partials,
-                      uint8_t *dict, uint32_t dict_cap, hipStream_t s)
-{
-    if (len <= 0) return;
-    const int32_t words = (int32_t)(((int64_t)len + 31) / 32);
-    if (dict_cap < rank_values_off((uint32_t)words)) fail(SDB_ERR_RUNTIME, "rank dictionary buffer too small");
-    const uint32_t cap_vals = (dict_cap - rank_values_off((uint32_t)words)) / 2u;
-    // the bitmap kernel's blocks each counted one run of 32 words when its
-    // grid covers the table without wrapping (below 2^21 slots; dictionaries
-    // are built for tables far smaller)
-    static_assert(64 * BITS_GROUPS * (BLOCK / 64) == 32 * RANK_PART_WORDS, "one bitmap block per 32 words");
-    const uint32_t ranges = (uint32_t)(((int64_t)words + RANK_PART_WORDS - 1) / RANK_PART_WORDS);
-    if (!partials || ranges != bits_partials(len))
-        fail(SDB_ERR_RUNTIME, "rank dictionary: the bitmap's per-block counts do not cover 32 words each");
-    hipLaunchKernelGGL(k_rank_dict_parts, dim3(ranges), dim3(64), 0, s, bits, words, partials, vals, (uint32_t)len,
-                       dict, cap_vals);
-    check_launch("rank_dict");
 }
 
 void launch_batch_masks(const FMaskCol *cols, int ncols, uint32_t max_len, const FMaskEntry *ents, hipStream_t s)

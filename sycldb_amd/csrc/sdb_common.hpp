@@ -106,4 +106,21 @@ struct StatsParts {
 };
 void launch_stats_reduce(const StatsParts &p, uint32_t *dst, hipStream_t s);
 
+// One compact table to build.  dict (or null): the rank dictionary
+// (FV_RANK16 layout, capacity dict_cap bytes) of its presence bitmap and
+// 16-bit values is built too.
+struct CompactJob {
+    const void *ht;
+    bool pairs;          // (flag, value) pairs, else uint8 keys
+    int32_t len, vmin;
+    uint32_t *bits;
+    uint16_t *vals;      // 16-bit value offsets, or null
+    uint32_t *partials, *bad;
+    uint8_t *dict;
+    uint32_t dict_cap;
+};
+// Builds them in one launch per COMPACT_JOBS tables (two with dictionaries);
+// returns the number of launches.
+int launch_compact_tables(const CompactJob *jobs, size_t njobs, hipStream_t s);
+
 } // namespace sdb

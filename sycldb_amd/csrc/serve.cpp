@@ -213,7 +213,7 @@ struct Server {
         r.batch_size = 1;
         r.status = guarded([&] {
             SDB_HIP(hipSetDevice(eng.device));
-            eng.mm->reset(eng.stream);
+            eng.begin_execution();
             r.result = execute_ddor_plan(eng, r.plan);
         });
         r.ran = true;

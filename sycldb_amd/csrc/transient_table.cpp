@@ -195,6 +195,7 @@ void TransientTable::execute_pending_kernels(bool dead_after)
     }
     ctx.virgin_live = virgin_live;
     const uint64_t nseg = segment_num();
+    ctx.whole_table = nseg == 1;
     for (const auto &phase : pending_kernels_)
         if (phase.size() != nseg) throw std::runtime_error("Pending kernels segment number mismatch.");
     for (uint64_t s = 0; s < nseg; s++) {
@@ -572,8 +573,9 @@ std::tuple<int32_t *, int32_t, int32_t> TransientTable::build_key_vals_hash_tabl
 // for a full join when the values fit, with their rank dictionary when small
 // enough for LDS), plus the fraction of set slots, which orders predicates.
 // Results never depend on them: a bit is set exactly when the reference
-// table reports a match.  Only the launches happen here; the statistics are
-// read on first use (Engine::resolve_compact).
+// table reports a match.  The build is only queued here (Engine::flush_builds
+// launches it, with the other joins' builds); the statistics are read on first
+// use (Engine::resolve_compact).
 // The value layout of a pair table, from its number of set slots (or a bound
 // on it) and its overflow flag: the 16-bit values when they fit, with their
 // rank dictionary staged for `set` values when that fits its buffer.
@@ -599,9 +601,11 @@ static void settle_values(CompactState &c, uint32_t set, uint32_t overflow)
 // when the group-by column's range fits them (vmax - vmin < 0xFFFF), so no
 // value overflows; its set slots are at most the build rows (each inserts one
 // key), so a dictionary sized for that many values holds them all.
+// `staged`: the probing program may stage the table in LDS (a captured one
+// never does, so it gets no rank dictionary).
 static std::shared_ptr<CompactState> build_compact(Engine &eng, const void *ht, bool pairs, int32_t ht_min,
                                                    int32_t ht_max, int32_t vmin, int32_t vmax, uint64_t build_rows,
-                                                   float est_sel = -1.0f)
+                                                   bool staged, float est_sel)
 {
     auto c = std::make_shared<CompactState>();
     const int64_t len = (int64_t)ht_max - ht_min + 1;
@@ -612,12 +616,7 @@ static std::shared_ptr<CompactState> build_compact(Engine &eng, const void *ht, 
     uint32_t *stats = eng.mm->alloc_zero<uint32_t>(1 + (uint64_t)nparts);
     const bool narrow = pairs && (int64_t)vmax - vmin < 0xFFFF;
     uint16_t *vals = narrow ? eng.mm->alloc<uint16_t>((uint64_t)len) : nullptr;
-    if (pairs)
-        launch_bits_from_pairs(static_cast<const int32_t *>(ht), (int32_t)len, bits, vals, vmin, stats + 1, stats,
-                               eng.stream);
-    else
-        launch_bits_from_keys(static_cast<const uint8_t *>(ht), (int32_t)len, bits, stats + 1, eng.stream);
-    eng.launches++;
+    CompactJob job{ht, pairs, (int32_t)len, vmin, bits, vals, stats + 1, stats, nullptr, 0};
     c->bits = bits;
     c->stats = stats;
     c->nparts = nparts;
@@ -628,12 +627,13 @@ static std::shared_ptr<CompactState> build_compact(Engine &eng, const void *ht, 
     c->build_rows = build_rows;
     // the dictionary goes into a buffer of the largest size staged in LDS;
     // whether it is used depends on the number of set slots
-    if (narrow && words <= 0xFFFFu && rank_values_off((uint32_t)words) < F_RANK_DICT_MAX) {
+    if (staged && narrow && words <= 0xFFFFu && rank_values_off((uint32_t)words) < F_RANK_DICT_MAX) {
         c->dict = eng.mm->alloc<uint8_t>(F_RANK_DICT_MAX);
         c->dict_cap = F_RANK_DICT_MAX;
-        launch_rank_dict(bits, (int32_t)len, vals, stats + 1, c->dict, c->dict_cap, eng.stream);
-        eng.launches++;
+        job.dict = c->dict;
+        job.dict_cap = c->dict_cap;
     }
+    eng.compact_jobs.push_back(job);
     if (est_sel >= 0.0f) {
         c->sel = std::min(1.0f, est_sel);
         if (pairs) settle_values(*c, (uint32_t)std::min<uint64_t>(build_rows, (uint64_t)len), 0);
@@ -644,8 +644,24 @@ static std::shared_ptr<CompactState> build_compact(Engine &eng, const void *ht, 
     return c;
 }
 
+void Engine::flush_builds()
+{
+    if (!dim_jobs.empty()) launches += launch_dim_builds(dim_jobs.data(), dim_jobs.size(), stream);
+    dim_jobs.clear();
+    if (!compact_jobs.empty()) launches += launch_compact_tables(compact_jobs.data(), compact_jobs.size(), stream);
+    compact_jobs.clear();
+}
+
+void Engine::begin_execution()
+{
+    mm->reset(stream);
+    dim_jobs.clear(); // of an execution that ended in an error
+    compact_jobs.clear();
+}
+
 void Engine::resolve_compact()
 {
+    flush_builds();
     std::vector<std::shared_ptr<CompactState>> todo;
     for (auto &w : pending_compact)
         if (auto c = w.lock())
@@ -694,6 +710,7 @@ void TransientTable::apply_join(TransientTable &right, const RelNode &rel)
         right_column >= (int64_t)right.current_columns_.size())
         throw std::invalid_argument("Invalid column indices in join condition.");
     Column *probe = col(left_column, "join probe");
+    const bool staged = !(eng_.capture.active && name_ == eng_.capture.table);
 
     if (rel.joinType == "semi") {
         auto ht = right.build_keys_hash_table((int)right_column);
@@ -702,7 +719,7 @@ void TransientTable::apply_join(TransientTable &right, const RelNode &rel)
         std::shared_ptr<CompactState> ct;
         if (eng_.fusion)
             ct = build_compact(eng_, std::get<0>(ht), false, std::get<1>(ht), std::get<2>(ht), 0, 0, right.nrows_,
-                               join_estimates() ? right.est_kept_ : -1.0f);
+                               staged, join_estimates() ? right.est_kept_ : -1.0f);
         std::vector<KernelBundle> ops(segment_num());
         for (uint64_t s = 0; s < segment_num(); s++) {
             const uint64_t off = s * eng_.segment_size;
@@ -739,7 +756,7 @@ void TransientTable::apply_join(TransientTable &right, const RelNode &rel)
     std::shared_ptr<CompactState> ct;
     if (eng_.fusion)
         ct = build_compact(eng_, std::get<0>(ht), true, std::get<1>(ht), std::get<2>(ht), gb_mm.first, gb_mm.second,
-                           right.nrows_, join_estimates() ? right.est_kept_ : -1.0f);
+                           right.nrows_, staged, join_estimates() ? right.est_kept_ : -1.0f);
     std::vector<KernelBundle> ops(segment_num());
     for (uint64_t s = 0; s < segment_num(); s++) {
         const uint64_t off = s * eng_.segment_size;
