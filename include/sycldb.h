@@ -518,6 +518,16 @@ uint64_t sdb_result_selected(const sdb_result *r);
  * values at those rows (sdb_result_selected values, int32 or uint64). */
 int sdb_result_selected_rows(const sdb_result *r, uint64_t *host);
 int sdb_result_col_copy_selected(const sdb_result *r, int c, void *host);
+/* The same in two calls: what a result holds, and its selected rows in one
+ * buffer of selected_bytes bytes: the row numbers (uint64), then each column's
+ * values (int32 or uint64) from the next multiple of 8 bytes on.  Bit c of
+ * u64_cols: column c (below 64) holds uint64 sums. */
+typedef struct sdb_result_info {
+    uint64_t nrows, selected, selected_bytes, u64_cols;
+    int ncols;
+} sdb_result_info;
+int sdb_result_describe(const sdb_result *r, sdb_result_info *info);
+int sdb_result_selected_copy(const sdb_result *r, void *host);
 /* Writes the .res text of executor/result_writer.cpp:41-67 (selected rows,
  * space-separated, int32 keys and uint64 sums) to `path`. */
 int sdb_result_write(const sdb_result *r, const char *path);

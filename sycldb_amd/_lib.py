@@ -81,6 +81,14 @@ class RequestInfo(ctypes.Structure):
                 ("batch_size", ctypes.c_int)]
 
 
+class ResultInfo(ctypes.Structure):
+    _fields_ = [("nrows", ctypes.c_uint64),
+                ("selected", ctypes.c_uint64),
+                ("selected_bytes", ctypes.c_uint64),
+                ("u64_cols", ctypes.c_uint64),
+                ("ncols", ctypes.c_int)]
+
+
 # sdb_op_kind (KernelType order)
 (OP_EMPTY, OP_LOGICAL, OP_SELECT_COL, OP_SELECT_LIT, OP_FILL, OP_BINOP_CC, OP_BINOP_LC, OP_BINOP_CL,
  OP_BUILD_KEYS, OP_PROBE_SEMI, OP_BUILD_KEYVALS, OP_PROBE_FULL, OP_SUM, OP_GROUPBY) = range(14)
@@ -182,6 +190,8 @@ SIGNATURES = {
     "sdb_result_selected": (U64, [P]),
     "sdb_result_selected_rows": (INT, [P, P]),
     "sdb_result_col_copy_selected": (INT, [P, INT, P]),
+    "sdb_result_describe": (INT, [P, P]),
+    "sdb_result_selected_copy": (INT, [P, P]),
     "sdb_result_write": (INT, [P, CSTR]),
     "sdb_result_destroy": (None, [P]),
     "sdb_plan_dag_order": (INT, [CSTR, P, INT, ctypes.POINTER(INT)]),

@@ -474,9 +474,10 @@ ExecutionInfo parse_execution_info(const PlanResult &plan);     // preprocessing
 // `sel` holds the selected rows in ascending order and every column only its
 // values at those rows; flags are empty and unselected rows read as 0 (the
 // sums of unselected group-by slots are 0, their keys are never written).
+// `listed`: `sel` holds the selected rows of a dense table too.
 struct ResultTable {
     uint64_t nrows = 0;
-    bool sparse = false;
+    bool sparse = false, listed = false;
     std::vector<uint8_t> flags;
     std::vector<uint32_t> sel;
     struct Col {
@@ -491,6 +492,10 @@ struct ResultTable {
     void col_to(int c, void *host) const;               // nrows values
     void selected_rows_to(uint64_t *host) const;        // selected() row ids
     void col_selected_to(int c, void *host) const;      // selected() values
+    void list_selected();                               // fills sel of a dense table
+    // row ids (uint64), then every column's values, each part 8-byte aligned
+    uint64_t selected_bytes() const;
+    void selected_to(uint8_t *host) const;
 };
 
 // The final table of a plan, on the device (valid until the allocator resets).

@@ -725,6 +725,28 @@ int sdb_result_col_copy_selected(const sdb_result *r, int c, void *host)
     });
 }
 
+int sdb_result_describe(const sdb_result *r, sdb_result_info *info)
+{
+    return guarded([&] {
+        require(r && info, "null argument");
+        info->nrows = r->t.nrows;
+        info->selected = r->t.selected();
+        info->selected_bytes = r->t.selected_bytes();
+        info->ncols = (int)r->t.cols.size();
+        info->u64_cols = 0;
+        for (size_t c = 0; c < r->t.cols.size() && c < 64; c++)
+            if (r->t.cols[c].is_u64) info->u64_cols |= 1ull << c;
+    });
+}
+
+int sdb_result_selected_copy(const sdb_result *r, void *host)
+{
+    return guarded([&] {
+        require(r && host, "null argument");
+        r->t.selected_to(static_cast<uint8_t *>(host));
+    });
+}
+
 int sdb_result_write(const sdb_result *r, const char *path)
 {
     return guarded([&] {

@@ -487,6 +487,8 @@ std::vector<ResultTable> copy_results(Engine &eng, const std::vector<FinalTable>
     if (!st.empty()) eng.launches += launch_sparse_tables(st.data(), st.size(), eng.stream);
     copies.wait(eng);
     copies.deliver(host);
+    for (ResultTable &res : out)
+        if (!res.sparse && res.nrows < RESULT_SPARSE_MIN_ROWS) res.list_selected();
     for (size_t j = 0; j < staged.size(); j++) {
         ResultTable &res = out[staged[j]];
         const SparseTable &s = st[j];
@@ -539,9 +541,43 @@ std::vector<ResultTable> copy_results(Engine &eng, const std::vector<FinalTable>
 
 ResultTable copy_result(Engine &eng, const FinalTable &t) { return std::move(copy_results(eng, {t})[0]); }
 
+void ResultTable::list_selected()
+{
+    uint64_t r = 0;
+    for (; r + 8 <= flags.size(); r += 8) { // mostly empty group-by slots: eight at a time
+        uint64_t w;
+        std::memcpy(&w, flags.data() + r, 8);
+        if (!w) continue;
+        for (uint64_t k = r; k < r + 8; k++)
+            if (flags[k]) sel.push_back((uint32_t)k);
+    }
+    for (; r < flags.size(); r++)
+        if (flags[r]) sel.push_back((uint32_t)r);
+    listed = true;
+}
+
+uint64_t ResultTable::selected_bytes() const
+{
+    const uint64_t k = selected();
+    uint64_t b = 8 * k;
+    for (const Col &c : cols) b += ((c.is_u64 ? 8 : 4) * k + 7) / 8 * 8;
+    return b;
+}
+
+void ResultTable::selected_to(uint8_t *host) const
+{
+    const uint64_t k = selected();
+    selected_rows_to(reinterpret_cast<uint64_t *>(host));
+    host += 8 * k;
+    for (size_t c = 0; c < cols.size(); c++) {
+        col_selected_to((int)c, host);
+        host += ((cols[c].is_u64 ? 8 : 4) * k + 7) / 8 * 8;
+    }
+}
+
 uint64_t ResultTable::selected() const
 {
-    if (sparse) return sel.size();
+    if (sparse || listed) return sel.size();
     uint64_t n = 0;
     for (uint8_t f : flags) n += f != 0;
     return n;
@@ -578,7 +614,7 @@ void ResultTable::col_to(int c, void *host) const
 
 void ResultTable::selected_rows_to(uint64_t *host) const
 {
-    if (sparse) {
+    if (sparse || listed) {
         for (size_t j = 0; j < sel.size(); j++) host[j] = sel[j];
         return;
     }
@@ -593,6 +629,13 @@ void ResultTable::col_selected_to(int c, void *host) const
     if (sparse) {
         if (col.is_u64) std::memcpy(host, col.u64.data(), col.u64.size() * 8);
         else std::memcpy(host, col.i32.data(), col.i32.size() * 4);
+        return;
+    }
+    if (listed) {
+        if (col.is_u64)
+            for (size_t j = 0; j < sel.size(); j++) static_cast<uint64_t *>(host)[j] = col.u64[sel[j]];
+        else
+            for (size_t j = 0; j < sel.size(); j++) static_cast<int32_t *>(host)[j] = col.i32[sel[j]];
         return;
     }
     uint64_t j = 0;

@@ -28,32 +28,33 @@ class Result:
         lib = L.lib
         self._h = ctypes.c_void_p(handle.value if isinstance(handle, ctypes.c_void_p) else handle)
         self._fin = weakref.finalize(self, lib.sdb_result_destroy, self._h)
-        self.nrows = int(lib.sdb_result_nrows(self._h))
-        self._ncols = int(lib.sdb_result_ncols(self._h))
-        self._is_u64 = None
+        info = L.ResultInfo()
+        L.check(lib.sdb_result_describe(self._h, ctypes.byref(info)))
+        self._info = info
+        self.nrows = info.nrows
         self._selected = None
         self._flags = None
         self._columns = None
 
     def _u64(self):
-        if self._is_u64 is None:
-            self._is_u64 = [L.lib.sdb_result_col_is_u64(self._h, c) == 1 for c in range(self._ncols)]
-        return self._is_u64
+        info = self._info
+        if info.ncols > 64:
+            return [L.lib.sdb_result_col_is_u64(self._h, c) == 1 for c in range(info.ncols)]
+        return [info.u64_cols >> c & 1 == 1 for c in range(info.ncols)]
 
     def _fetch_selected(self):
         if self._selected is None:
-            lib = L.lib
-            k = int(lib.sdb_result_selected(self._h))
-            rows = np.zeros(k, dtype=np.uint64)
+            # one call for the row numbers and every column's values
+            k = self._info.selected
+            buf = np.empty(self._info.selected_bytes, np.uint8)
             if k:
-                L.check(lib.sdb_result_selected_rows(self._h, rows.ctypes.data_as(ctypes.c_void_p)))
-            cols = []
-            for c, u64 in enumerate(self._u64()):
-                arr = np.zeros(k, dtype=np.uint64 if u64 else np.int32)
-                if k:
-                    L.check(lib.sdb_result_col_copy_selected(self._h, c, arr.ctypes.data_as(ctypes.c_void_p)))
-                cols.append(arr)
-            self._selected = (rows, cols)
+                L.check(L.lib.sdb_result_selected_copy(self._h, buf.ctypes.data))
+            at, cols = 8 * k, []
+            for u64 in self._u64():
+                end = at + (8 if u64 else 4) * k
+                cols.append(buf[at:end].view(np.uint64 if u64 else np.int32))
+                at = (end + 7) // 8 * 8
+            self._selected = (buf[:8 * k].view(np.uint64), cols)
         return self._selected
 
     @property
