@@ -483,6 +483,27 @@ bool hash_groupby_enabled()
     return v;
 }
 
+// The groups a group-by is expected to meet: a key that a full join brought in
+// takes about the share of its range that the join's build side kept (a filter
+// on a column of the key's own hierarchy, as every star-join query has it),
+// any other key its whole range.
+double expected_groups(const std::vector<Draft> &d, const FGroup &g)
+{
+    double groups = 1.0;
+    for (int j = 0; j < g.k; j++) {
+        double keep = 1.0;
+        for (const Draft &D : d)
+            if (g.key_reg[j] >= 0 && D.I.vout == g.key_reg[j] && (D.I.kind == FK_PROBE_BITS || D.I.kind == FK_PROBE_FULL))
+                keep = std::min(1.0, std::max(0.0, (double)D.sel));
+        groups *= std::max(1.0, (double)g.range[j] * keep);
+    }
+    return groups;
+}
+// More groups than this leave the LDS hash crowded: most rows then search it in
+// vain (32 slots) and go to the global arrays all the same.  q3.x by city over
+// 30M rows (15,000 groups): the kernel 196 us through the hash, 182 without.
+constexpr double HASH_MAX_GROUPS = 4.0 * F_HASH_CAP;
+
 // Columns the kernel prefetches.  A lazily loaded column costs the whole
 // wave a dependent memory round trip whenever any of its lanes needs it, which
 // for 64 lanes x 4 rows is nearly always, so every column read is prefetched
@@ -810,8 +831,10 @@ bool KernelBundle::build_program(const ExecContext &ctx, FProgram &p) const
             // modulo): LDS copies (dense for small ranges, hashed otherwise)
             // with an exact flush
             fits = fits && exact == g.prod && g.prod <= 0x80000000ull;
+            G.exact = fits;
             G.lds = !fits ? FG_GLOBAL : (g.prod <= F_DENSE_MAX ? FG_DENSE_LDS : FG_HASH_LDS);
-            if (G.lds == FG_HASH_LDS && !hash_groupby_enabled()) G.lds = FG_GLOBAL;
+            if (G.lds == FG_HASH_LDS && (!hash_groupby_enabled() || expected_groups(d, G) > HASH_MAX_GROUPS))
+                G.lds = FG_GLOBAL;
             group_area = G.lds == FG_DENSE_LDS ? (uint32_t)(g.prod * 8 + (g.prod + 31) / 32 * 4 + 16)
                          : G.lds == FG_HASH_LDS ? F_HASH_CAP * 12u + 16u
                                                 : 0u;

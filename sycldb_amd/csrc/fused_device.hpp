@@ -114,10 +114,13 @@ __device__ __forceinline__ void gb_row_mode(const FGroup &g, uint8_t *lds, const
             // table crowded: fall through to the global update
         }
     }
-    const uint64_t s64 = (uint64_t)(int64_t)(int32_t)hash % g.prod;
-    // a slot already marked needs no exchange (a plain read; a stale 0 just
-    // leads to the exchange, which decides)
-    if (__hip_atomic_load(&g.seen[s64], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0u &&
+    // an in-range row of exactly multiplying key ranges has its slot already;
+    // the 64-bit remainder costs some 150 instructions
+    uint64_t s64 = hash;
+    if (!(in_range && (MODE != FG_GLOBAL || g.exact))) s64 = (uint64_t)(int64_t)(int32_t)hash % g.prod;
+    // a slot already marked needs no exchange: a read that may come from this
+    // XCD's L2 (a stale 0 just leads to the exchange, which decides)
+    if (__hip_atomic_load(&g.seen[s64], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) == 0u &&
         atomicExch(&g.seen[s64], 1u) == 0u) {
 #pragma unroll
         for (int j = 0; j < F_MAX_KEYS; j++)

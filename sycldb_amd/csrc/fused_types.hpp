@@ -108,6 +108,8 @@ struct FGroup {
     uint64_t prod;
     uint32_t lds_off;          // byte offset of the LDS aggregation area
     uint32_t hash_cap;         // FG_HASH_LDS: slots (power of two)
+    uint32_t exact;            // the key ranges multiply to prod (< 2^31): an in-range
+                               // row's slot is its index, no remainder
 };
 
 // Initial value of a flag register.  FF_UNDEF is 0 so that registers a

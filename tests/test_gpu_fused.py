@@ -4,6 +4,7 @@ import pytest
 
 pytestmark = pytest.mark.gpu
 
+from oracle import datagen, plan_oracle as PO  # noqa: E402
 from sycldb_amd import plans as PL  # noqa: E402
 from sycldb_amd import schema as S  # noqa: E402
 from sycldb_amd.engine import Engine  # noqa: E402
@@ -32,3 +33,20 @@ def test_presence_filter_of_a_wide_probe():
                 plan = PL.t2_plan(part, 2)
                 fused, unfused = _both(eng, plan)
                 assert fused == unfused and len(fused) > 0
+
+
+# The groups a group-by is expected to meet decide its form: 6 x 10 x 10 in
+# the LDS hash, 6 x 10 x 50 crowding it, 6 x 50 x 50 straight to the global
+# arrays; a build side with keys outside the group's range (the slot's
+# remainder) stays with the general form.
+@pytest.mark.parametrize("cust,supp", [(("nation", 6), ("nation", 6)), (("nation", 6), ("region", 1)),
+                                       (("region", 1), ("region", 3))])
+@pytest.mark.parametrize("codegen", ["compile", "interpret"])
+def test_groupby_forms(cust, supp, codegen):
+    from sycldb_amd.engine import Engine
+    plan = PL.build("t3", cust=cust, supp=supp, date=("year_range", 1992, 1997), group="city")
+    tables = datagen.generate_tables(S, 300_007, 45)
+    want = PO.execute_plan(plan, tables).rows()
+    with Engine(codegen=codegen) as eng:
+        eng.generate(300_007, 45)
+        assert eng.execute(plan).rows() == want and len(want) > 100
