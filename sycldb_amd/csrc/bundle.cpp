@@ -116,6 +116,8 @@ void KernelBundle::execute(const ExecContext &ctx) const
             if (eng.codegen == SDB_CODEGEN_AUTO && !eng.unroll && ctx.whole_table && !stores_part &&
                 !eng.profiles(ctx.table) && dim_job(p, n, job)) {
                 eng.dim_jobs.push_back(job);
+                // a batch's first launches run while its later plans are walked
+                if (eng.dim_jobs.size() >= DIM_JOBS) eng.flush_builds();
                 if (stores_whole) ctx.virgin_filled = true;
                 eng.mark("queued");
                 return;

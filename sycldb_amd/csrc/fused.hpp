@@ -95,8 +95,9 @@ void set_batch_trials(bool on);
 // of every CU free, so that one engine's kernels run beside another's
 // batched scan instead of behind it.
 void set_batch_waves_per_cu(int cap);
-// Builds the mask tables of a batched launch (ops.hip).
-void launch_batch_masks(const FMaskCol *cols, int ncols, uint32_t max_len, const FMaskEntry *ents, hipStream_t s);
+// Builds the mask tables of a batched launch (ops.hip).  cols: device memory;
+// lens: their table lengths, on the host.
+void launch_batch_masks(const FMaskCol *cols, const uint32_t *lens, int ncols, const FMaskEntry *ents, hipStream_t s);
 // Builds the rank dictionaries of some of them, after the tables (ops.hip).
 void launch_batch_dict(const FMaskDict *dicts, int ndicts, hipStream_t s);
 // Compiles (no device needed) a batched kernel over the coverage programs.

@@ -3256,7 +3256,7 @@ void launch_fused_batch(const std::vector<FProgram> &in, int64_t n, hipStream_t 
     std::vector<uint32_t> mshift(std::max(nmask, 1), 0), mwbytes(std::max(nmask, 1), 4);
     std::vector<uint32_t> mlds(std::max(nmask, 1), 0), mdict(std::max(nmask, 1), 0);
     std::vector<const uint8_t *> mdg(std::max(nmask, 1), nullptr);
-    uint32_t max_len = 0;
+    std::vector<uint32_t> mask_lens;
     {
         size_t at = 16, ei = 0;
         for (size_t ci = 0; ci < b.masks.size(); ci++) {
@@ -3278,7 +3278,7 @@ void launch_fused_batch(const std::vector<FProgram> &in, int64_t n, hipStream_t 
                 probing |= 1u << e.bit;
             }
             std::memcpy(host + off_cols + ci * sizeof(FMaskCol), &c, sizeof(FMaskCol));
-            max_len = std::max(max_len, c.len);
+            mask_lens.push_back(c.len);
             const int mi = (int)(std::find(b.mask_slots.begin(), b.mask_slots.end(), m.slot) - b.mask_slots.begin());
             mtab[mi] = c.tab;
             mlo[mi] = c.lo;
@@ -3377,7 +3377,7 @@ void launch_fused_batch(const std::vector<FProgram> &in, int64_t n, hipStream_t 
                       HIP_LAUNCH_PARAM_END};
     auto enqueue = [&]() {
         SDB_HIP(hipMemcpyAsync(dblock, host, copy_bytes, hipMemcpyHostToDevice, s));
-        if (nmask > 0 && !b.masks.empty()) launch_batch_masks(d_cols, (int)b.masks.size(), max_len, d_ents, s);
+        if (nmask > 0 && !b.masks.empty()) launch_batch_masks(d_cols, mask_lens.data(), (int)b.masks.size(), d_ents, s);
         launch_batch_dict(d_dicts, ndicts, s);
         SDB_HIP(hipModuleLaunchKernel(k.fn, grid, 1, 1, shape.block, 1, 1, b.lds, s, nullptr, config));
     };
@@ -3401,9 +3401,10 @@ void launch_fused_batch(const std::vector<FProgram> &in, int64_t n, hipStream_t 
         // graph serves launches with the same geometry and the same
         // arguments; the programs and mask descriptors travel in the copy
         char head[256];
-        snprintf(head, sizeof(head), "%p/%u/%d/%u/%zu/%u/%zu/%p/%p/", (void *)k.fn, grid, shape.block, b.lds, copy_bytes,
-                 max_len, b.masks.size(), (void *)dblock, (void *)host);
+        snprintf(head, sizeof(head), "%p/%u/%d/%u/%zu/%zu/%p/%p/", (void *)k.fn, grid, shape.block, b.lds, copy_bytes,
+                 b.masks.size(), (void *)dblock, (void *)host);
         std::string topo(head);
+        topo.append(reinterpret_cast<const char *>(mask_lens.data()), 4 * mask_lens.size()); // the mask build's grid
         topo.append(reinterpret_cast<const char *>(args.data()), args.size());
         auto hit = std::find_if(G->execs.begin(), G->execs.end(), [&](const std::pair<std::string, hipGraphExec_t> &e) {
             return e.first == topo;
@@ -3454,7 +3455,7 @@ void launch_fused_batch(const std::vector<FProgram> &in, int64_t n, hipStream_t 
     // a tuning trial: the kernel alone, timed with HIP events; compared per
     // row and program, since batches of one library differ in size
     SDB_HIP(hipMemcpyAsync(dblock, host, copy_bytes, hipMemcpyHostToDevice, s));
-    if (nmask > 0 && !b.masks.empty()) launch_batch_masks(d_cols, (int)b.masks.size(), max_len, d_ents, s);
+    if (nmask > 0 && !b.masks.empty()) launch_batch_masks(d_cols, mask_lens.data(), (int)b.masks.size(), d_ents, s);
     launch_batch_dict(d_dicts, ndicts, s);
     hipEvent_t ea, eb;
     SDB_HIP(hipEventCreate(&ea));

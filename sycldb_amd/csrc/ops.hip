@@ -1360,33 +1360,94 @@ template <int N> __global__ void __launch_bounds__(64) k_rank_dicts(RankJobs<N> 
 }
 
 // ------------------------------------------------------- batch probe masks
-// One thread per key of a masked fact column (blockIdx.y = column): the key's
-// word starts with every program's bit and loses the bit of each program one
-// of whose probes on the column fails for the key -- the probe's own test
-// (range check, then the table entry: FilterJoinKernel / FullJoinKernel,
-// kernels/join.hpp:129-160, 256-300).
-__global__ void __launch_bounds__(BLOCK) k_batch_masks(const FMaskCol *cols, const FMaskEntry *ents)
+// Every key of a masked fact column: the key's word starts with every
+// program's bit and loses the bit of each program one of whose probes on the
+// column fails for the key -- the probe's own test (range check, then the
+// table entry: FilterJoinKernel / FullJoinKernel, kernels/join.hpp:129-160,
+// 256-300).
+//
+// Four consecutive keys per thread (their bits of a bitmap lie in one or two
+// words, their windows in one store), 1,024 per block; the block's entries
+// come through LDS, and the bitmap words of four entries load together.
+constexpr uint32_t MASK_KEYS = 4 * BLOCK;
+constexpr uint32_t MASK_ENTS = 64; // entries in LDS at a time
+constexpr int MASK_GROUP = 4;
+struct MaskGrid {
+    uint32_t first[F_MASK_MAX_COLS]; // first block of each column (unused: UINT32_MAX)
+};
+
+// bit k: whether the probe passes for key + k
+__device__ __forceinline__ uint32_t mask_probe(const FMaskEntry &E, int32_t key)
 {
-    const FMaskCol c = cols[blockIdx.y];
-    for (uint32_t i = blockIdx.x * BLOCK + threadIdx.x; i < c.len; i += gridDim.x * BLOCK) {
-        const int32_t key = (int32_t)((uint32_t)c.lo + i);
-        uint32_t w = c.full;
-        for (uint32_t e = c.first; e < c.first + c.count; e++) {
-            const FMaskEntry E = ents[e];
-            bool pass = key >= E.ht_min && key <= E.ht_max;
-            if (pass) {
-                const uint32_t s = slot_of(key, E.ht_min);
-                if (E.kind == FM_BITS) pass = (reinterpret_cast<const uint32_t *>(E.ht)[s >> 5] >> (s & 31)) & 1u;
-                else if (E.kind == FM_SEMI) pass = reinterpret_cast<const uint8_t *>(E.ht)[s] != 0;
-                else pass = reinterpret_cast<const int2 *>(E.ht)[s].x == 1;
-            }
-            if (!pass) w &= ~(1u << E.bit);
-        }
-        const uint32_t v = w >> c.shift;
-        if (c.wbytes == 1) c.tab[i] = (uint8_t)v;
-        else if (c.wbytes == 2) reinterpret_cast<uint16_t *>(c.tab)[i] = (uint16_t)v;
-        else reinterpret_cast<uint32_t *>(c.tab)[i] = v;
+    uint32_t m = 0;
+    for (int k = 0; k < 4; k++) {
+        const int32_t x = (int32_t)((uint32_t)key + (uint32_t)k);
+        if (x < E.ht_min || x > E.ht_max) continue;
+        const uint32_t s = slot_of(x, E.ht_min);
+        bool pass;
+        if (E.kind == FM_BITS) pass = (reinterpret_cast<const uint32_t *>(E.ht)[s >> 5] >> (s & 31)) & 1u;
+        else if (E.kind == FM_SEMI) pass = reinterpret_cast<const uint8_t *>(E.ht)[s] != 0;
+        else pass = reinterpret_cast<const int2 *>(E.ht)[s].x == 1;
+        m |= (uint32_t)pass << k;
     }
+    return m;
+}
+
+__global__ void __launch_bounds__(BLOCK) k_batch_masks(const FMaskCol *__restrict__ cols,
+                                                       const FMaskEntry *__restrict__ ents, MaskGrid grid)
+{
+    __shared__ FMaskEntry E[MASK_ENTS];
+    int j = 0;
+#pragma unroll
+    for (int k = 1; k < F_MASK_MAX_COLS; k++) j += blockIdx.x >= grid.first[k];
+    const FMaskCol c = cols[j];
+    const uint32_t i = (blockIdx.x - grid.first[j]) * MASK_KEYS + 4u * threadIdx.x;
+    const int32_t key = (int32_t)((uint32_t)c.lo + i);
+    uint32_t w[4] = {c.full, c.full, c.full, c.full};
+    for (uint32_t e0 = 0; e0 < c.count; e0 += MASK_ENTS) {
+        const uint32_t n = min(c.count - e0, MASK_ENTS);
+        __syncthreads();
+        for (uint32_t e = threadIdx.x; e < n; e += BLOCK) E[e] = ents[c.first + e0 + e];
+        __syncthreads();
+        if (i >= c.len) continue;
+        for (uint32_t e = 0; e < n; e += MASK_GROUP) {
+            uint32_t lo[MASK_GROUP], hi[MASK_GROUP], slot[MASK_GROUP];
+            bool whole[MASK_GROUP]; // a bitmap that holds all four keys
+#pragma unroll
+            for (int q = 0; q < MASK_GROUP; q++) {
+                const uint32_t at = min(e + q, n - 1u);
+                const uint32_t s = slot_of(key, E[at].ht_min), last = slot_of(E[at].ht_max, E[at].ht_min);
+                whole[q] = E[at].kind == FM_BITS && E[at].ht_min <= E[at].ht_max && s <= last && last - s >= 3u;
+                slot[q] = s;
+                lo[q] = hi[q] = 0;
+                if (whole[q]) {
+                    const uint32_t *bits = reinterpret_cast<const uint32_t *>(E[at].ht);
+                    lo[q] = bits[s >> 5];
+                    hi[q] = bits[(s + 3u) >> 5];
+                }
+            }
+#pragma unroll
+            for (int q = 0; q < MASK_GROUP; q++) {
+                if (e + q >= n) break;
+                const uint32_t pass = whole[q] ? __builtin_amdgcn_alignbit(hi[q], lo[q], slot[q] & 31u)
+                                               : mask_probe(E[e + q], key);
+#pragma unroll
+                for (int k = 0; k < 4; k++)
+                    if (!((pass >> k) & 1u)) w[k] &= ~(1u << E[e + q].bit);
+            }
+        }
+    }
+    if (i >= c.len) return;
+    // (the table is padded to 16 bytes: the last keys' windows store whole)
+#pragma unroll
+    for (int k = 0; k < 4; k++) w[k] >>= c.shift;
+    if (c.wbytes == 1)
+        *reinterpret_cast<uint32_t *>(c.tab + i) =
+            (w[0] & 0xffu) | (w[1] & 0xffu) << 8 | (w[2] & 0xffu) << 16 | (w[3] & 0xffu) << 24;
+    else if (c.wbytes == 2)
+        *reinterpret_cast<uint2 *>(c.tab + 2 * i) = make_uint2((w[0] & 0xffffu) | w[1] << 16, (w[2] & 0xffffu) | w[3] << 16);
+    else
+        *reinterpret_cast<uint4 *>(c.tab + 4 * (size_t)i) = make_uint4(w[0], w[1], w[2], w[3]);
 }
 
 // Rank dictionaries of batched mask tables (FMaskDict), one block per table.
@@ -1396,7 +1457,7 @@ __global__ void __launch_bounds__(BLOCK) k_batch_masks(const FMaskCol *cols, con
 // bit per key is whether the key's window is nonzero.  The exclusive counts
 // before each word are scanned across the block; then each thread reloads its
 // words' windows and writes every set key's window at its rank.
-constexpr int DICT_BLOCK = 256;
+constexpr int DICT_BLOCK = 1024;
 constexpr uint32_t DICT_MAX_WORDS = F_DICT_MAX_LEN / 32;
 
 template <uint32_t WB> __device__ void dict_bits(const FMaskDict &d, uint32_t words, uint32_t *sbits)
@@ -2244,11 +2305,19 @@ void launch_stats_reduce(const StatsParts &p, uint32_t *dst, hipStream_t s)
     check_launch("stats_reduce");
 }
 
-void launch_batch_masks(const FMaskCol *cols, int ncols, uint32_t max_len, const FMaskEntry *ents, hipStream_t s)
+void launch_batch_masks(const FMaskCol *cols, const uint32_t *lens, int ncols, const FMaskEntry *ents, hipStream_t s)
 {
-    if (ncols <= 0 || max_len == 0) return;
-    const unsigned gx = (unsigned)std::min<uint64_t>(((uint64_t)max_len + BLOCK - 1) / BLOCK, 4096);
-    hipLaunchKernelGGL(k_batch_masks, dim3(gx, (unsigned)ncols), dim3(BLOCK), 0, s, cols, ents);
+    if (ncols <= 0) return;
+    if (ncols > F_MASK_MAX_COLS) fail(SDB_ERR_RUNTIME, "batch masks: too many columns");
+    MaskGrid grid;
+    std::fill(std::begin(grid.first), std::end(grid.first), UINT32_MAX);
+    uint32_t blocks = 0;
+    for (int c = 0; c < ncols; c++) {
+        grid.first[c] = blocks;
+        blocks += (lens[c] + MASK_KEYS - 1) / MASK_KEYS;
+    }
+    if (!blocks) return;
+    hipLaunchKernelGGL(k_batch_masks, dim3(blocks), dim3(BLOCK), 0, s, cols, ents, grid);
     check_launch("batch_masks");
 }
 
