@@ -170,6 +170,37 @@ void KernelBundle::build_captured(Engine &eng, CapturedBundle &cb)
     dump_program(cb.p, cb.n, cb.table + " (captured)");
 }
 
+// The two flag buffers a chain of operators alternates between, when one can
+// take the place of both: every operator reads the one written last, and
+// nothing reads either afterwards.  (Flags read and written in place stay in
+// the caches: 60M rows, a selection 67 -> 50 us, a semi probe 70 -> 57.)
+static std::pair<const uint8_t *, uint8_t *> shared_flags(const std::vector<KernelData> &ks, const ExecContext &ctx)
+{
+    const std::pair<const uint8_t *, uint8_t *> none{nullptr, nullptr};
+    if (!ctx.flags_dead) return none;
+    const uint8_t *a = nullptr, *b = nullptr, *cur = nullptr;
+    for (const KernelData &k : ks) {
+        if (k.type == KernelType::EmptyKernel) continue;
+        if (!a && k.in_flags && k.out_flags && k.in_flags != k.out_flags) {
+            a = cur = k.in_flags;
+            b = k.out_flags;
+            if ((a < b ? b - a : a - b) < k.n) return none; // overlapping
+        }
+        if (!a) {
+            // before the pair is known, only a SEARCH's own flags may be used
+            if (k.in_flags != k.out_flags || !k.out_flags) return none;
+            continue;
+        }
+        auto stale = [&](const uint8_t *p) { return (p == a || p == b) && p != cur; };
+        if (stale(k.in_flags) || stale(k.local_flags)) return none;
+        if (k.out_flags == a || k.out_flags == b) {
+            if (k.in_flags != cur) return none;
+            cur = k.out_flags;
+        }
+    }
+    return {b, const_cast<uint8_t *>(a)};
+}
+
 void KernelBundle::execute_unfused(const ExecContext &ctx) const
 {
     hipStream_t s = ctx.stream;
@@ -185,8 +216,15 @@ void KernelBundle::execute_unfused(const ExecContext &ctx) const
         eng.launches++;
         ctx.virgin_filled = true;
     }
-    for (const KernelData &k : kernels_) {
-        if (k.type == KernelType::EmptyKernel) continue;
+    const auto shared = shared_flags(kernels_, ctx);
+    for (const KernelData &k0 : kernels_) {
+        if (k0.type == KernelType::EmptyKernel) continue;
+        KernelData k = k0;
+        if (shared.first) {
+            if (k.in_flags == shared.first) k.in_flags = shared.second;
+            if (k.local_flags == shared.first) k.local_flags = shared.second;
+            if (k.out_flags == shared.first) k.out_flags = shared.second;
+        }
         validate_kernel(k, eng.registry);
         Engine::ProfRec rec;
         const bool timed = eng.profiles(ctx.table);

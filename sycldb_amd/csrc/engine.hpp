@@ -246,6 +246,7 @@ struct ExecContext {
     // holding values (stored whole by a program, else filled)
     bool virgin_live = false;
     bool whole_table = false; // the table is one segment
+    bool flags_dead = false;  // nothing reads the table's flags after this bundle
 };
 
 // KernelBundle, models/execution.hpp:500-651: the operators queued for one

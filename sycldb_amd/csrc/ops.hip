@@ -153,8 +153,7 @@ template <int LOGIC> __device__ __forceinline__ uint32_t logical_bytes(uint32_t 
 // The same, 16 flags per thread and step (the three buffers 16-byte
 // aligned); the last n % 16 flags one per thread.
 template <int LOGIC>
-__global__ void __launch_bounds__(BLOCK) k_logical_vec(const uint8_t *__restrict__ in,
-                                                       const uint8_t *__restrict__ local, uint8_t *__restrict__ out,
+__global__ void __launch_bounds__(BLOCK) k_logical_vec(const uint8_t *in, const uint8_t *local, uint8_t *out,
                                                        int64_t n)
 {
     const int64_t nq = n >> 4;

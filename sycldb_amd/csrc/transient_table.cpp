@@ -196,6 +196,7 @@ void TransientTable::execute_pending_kernels(bool dead_after)
     ctx.virgin_live = virgin_live;
     const uint64_t nseg = segment_num();
     ctx.whole_table = nseg == 1;
+    ctx.flags_dead = dead_after && pending_kernels_.size() == 1;
     for (const auto &phase : pending_kernels_)
         if (phase.size() != nseg) throw std::runtime_error("Pending kernels segment number mismatch.");
     for (uint64_t s = 0; s < nseg; s++) {
