@@ -49,6 +49,21 @@ bool join_estimates()
     return on;
 }
 
+// Whether a join over `rows` rows gets compact tables.  Their two launches (and
+// the host's part in them) cost more than a short column's probes gain from
+// them: q3.x over 200,000 rows 72 us with them, 66 on the reference tables;
+// 3M rows 131 and 122; 6M rows 111 and 125.  A batch reads a table only to build
+// its masks and for the kept rows' values: 8 pipelines over 6M rows 449 and
+// 437 us, over 12M 501 and 481.  Forced launch forms and exact statistics keep
+// them at every size.
+constexpr uint64_t COMPACT_MIN_ROWS = 4 << 20, COMPACT_MIN_BATCH_ROWS = 16 << 20;
+
+bool compact_pays(const Engine &eng, uint64_t rows, bool captured)
+{
+    if (eng.codegen != SDB_CODEGEN_AUTO || eng.unroll || !join_estimates()) return true;
+    return rows >= (captured ? COMPACT_MIN_BATCH_ROWS : COMPACT_MIN_ROWS);
+}
+
 // Fraction of a uniformly distributed column in [mn, mx] a comparison keeps
 // (used only to order fused predicates, never for results).
 float estimate_cmp(int cmp, int32_t lit, std::pair<int32_t, int32_t> mm)
@@ -718,7 +733,7 @@ void TransientTable::apply_join(TransientTable &right, const RelNode &rel)
         ensure_secondary_flags();
         right.execute_pending_kernels(false);
         std::shared_ptr<CompactState> ct;
-        if (eng_.fusion)
+        if (eng_.fusion && compact_pays(eng_, nrows_, !staged))
             ct = build_compact(eng_, std::get<0>(ht), false, std::get<1>(ht), std::get<2>(ht), 0, 0, right.nrows_,
                                staged, join_estimates() ? right.est_kept_ : -1.0f);
         std::vector<KernelBundle> ops(segment_num());
@@ -735,6 +750,7 @@ void TransientTable::apply_join(TransientTable &right, const RelNode &rel)
             k.ht_max = std::get<2>(ht);
             if (ct) k.bits = ct->bits;
             k.compact = ct;
+            k.sel = std::min(1.0f, right.est_kept_);
             ops[s].add_kernel(k);
         }
         add_pending_kernels(std::move(ops));
@@ -755,7 +771,7 @@ void TransientTable::apply_join(TransientTable &right, const RelNode &rel)
     ensure_secondary_flags();
     right.execute_pending_kernels(false);
     std::shared_ptr<CompactState> ct;
-    if (eng_.fusion)
+    if (eng_.fusion && compact_pays(eng_, nrows_, !staged))
         ct = build_compact(eng_, std::get<0>(ht), true, std::get<1>(ht), std::get<2>(ht), gb_mm.first, gb_mm.second,
                            right.nrows_, staged, join_estimates() ? right.est_kept_ : -1.0f);
     std::vector<KernelBundle> ops(segment_num());
@@ -773,6 +789,7 @@ void TransientTable::apply_join(TransientTable &right, const RelNode &rel)
         k.ht_max = std::get<2>(ht);
         if (ct) k.bits = ct->bits;
         k.compact = ct;
+        k.sel = std::min(1.0f, right.est_kept_);
         k.vmin = gb_mm.first;
         nc.seg_min[s] = gb_mm.first; // models/models.hpp:1609-1610
         nc.seg_max[s] = gb_mm.second;

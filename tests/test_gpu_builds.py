@@ -55,3 +55,20 @@ def test_many_large_results_in_one_batch():
             got, _ = eng.execute_batch(plans)
             for g, p in zip(got, plans):
                 assert g.rows() == PO.execute_plan(p, tables).rows(), p
+
+
+@pytest.mark.parametrize("rows", [(4 << 20) - 1, 4 << 20, (16 << 20) - 1, 16 << 20])
+def test_probe_tables_by_rows(rows):
+    """Joins over fewer rows than these probe the reference tables, over more
+    the compact ones (alone from 4M rows on, batched from 16M): the results of
+    one kernel per operator."""
+    from sycldb_amd.engine import Engine
+    plans = [PL.build(t, **p) for t, p in PLANS]
+    with Engine() as eng:
+        eng.generate(rows, 45)
+        eng.set_fusion(False)
+        want = [eng.execute(p).rows() for p in plans]
+        eng.set_fusion(True)
+        assert [eng.execute(p).rows() for p in plans] == want
+        got, batched = eng.execute_batch(plans)
+        assert [g.rows() for g in got] == want and batched == len(plans)
