@@ -752,6 +752,10 @@ __global__ void __launch_bounds__(PROBE_BLOCK) k_probe_full_lds(const int32_t *_
     for (; tile < ntiles; tile += stride) {
         const int64_t t0 = tile * WT_ROWS;
         const uint32_t flagged = wt_mask(next);
+        uint32_t other = 0; // flags other than 0 and 1 become 1
+#pragma unroll
+        for (int j = 0; j < WT_CHUNKS; j++) other |= next[j] & 0xfefefefeu;
+        const bool odd = other != 0;
         const bool whole = t0 + WT_ROWS <= n;
         uint32_t slot[WT_CHUNKS][4];
 #pragma unroll
@@ -857,6 +861,8 @@ __global__ void __launch_bounds__(PROBE_BLOCK) k_probe_full_lds(const int32_t *_
         for (int j = 0; j < WT_CHUNKS; j++) {
             const int64_t r = wt_row(t0, lane, j);
             const uint32_t f = flag_bytes(hits >> (4 * j));
+            // in place, flags that stay as they are need no write
+            if (in == out && !__any(odd || (((hits ^ flagged) >> (4 * j)) & 15u))) continue;
             if (whole || r + 3 < n) *reinterpret_cast<uint32_t *>(out + r) = f;
             else
                 for (int k = 0; k < 4; k++)
