@@ -251,7 +251,7 @@ def group_by_aggregate(contents, agg_column, max, min, flags, col_len, col_num, 
 
 def count_true_flags(flags, length, stream=None):
     """count_true_flags, kernels/common.hpp:67-79 (synchronous)."""
-    out = torch.zeros(1, dtype=torch.int64, device=flags.device)
+    out = torch.empty(1, dtype=torch.int64, device=flags.device)  # zeroed by the count
     count_flags(flags, out, accumulate=False, n=length, stream=stream)
     return int(out.item())
 
