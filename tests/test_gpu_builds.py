@@ -72,3 +72,52 @@ def test_probe_tables_by_rows(rows):
         assert [eng.execute(p).rows() for p in plans] == want
         got, batched = eng.execute_batch(plans)
         assert [g.rows() for g in got] == want and batched == len(plans)
+
+
+@pytest.mark.parametrize("table,column,value", [("customer", 4, 6), ("supplier", 5, 1), ("customer", 4, 99)])
+def test_results_that_are_no_groupby(table, column, value):
+    """A filtered dimension as the result: 300,000 rows (not listed when they
+    arrive) and 20,000 (listed), some rows selected and none."""
+    import json
+    from sycldb_amd.engine import Engine
+    plan = json.loads(PL.to_json(PL.build("t3", cust=("nation", 6))))
+    scan, keep = dict(plan["rels"][1], id=0, tables=["ssb", table]), dict(plan["rels"][2], id=1)
+    keep["condition"]["operands"][0].update(input=column, name="$%d" % column)
+    keep["condition"]["operands"][1]["literal"]["value"] = value
+    tables = datagen.generate_tables(S, 1000, 45)
+    for rels in ([scan, keep], [scan]):
+        want = PO.execute_plan(dict(plan, rels=rels), tables).rows()
+        for fusion in (True, False):
+            with Engine(fusion=fusion) as eng:
+                eng.generate(1000, 45)
+                got = eng.execute(dict(plan, rels=rels))
+                assert len(got.selected_rows) == len(want) and got.rows() == want
+                assert int((got.flags != 0).sum()) == len(want)
+
+
+def test_batch_reads_more_columns_than_the_shared_scan_holds():
+    """A q3.x sum over each of the 17 fact columns (the scan holds 16): the
+    column past it is read from memory.  Then a batch over a few of them in
+    the same engine, and the first again."""
+    import json
+    import numpy as np
+    from sycldb_amd.engine import Engine
+    rows, seed = 120_003, 45
+    tables = datagen.generate_tables(S, rows, seed)
+    rng = np.random.default_rng(1)
+    for c in set(range(17)) - set(tables["lineorder"]):
+        tables["lineorder"][c] = rng.integers(-1000, 1000, rows).astype(np.int32)
+    plans = []
+    for c in range(17):
+        p = json.loads(PL.to_json(PL.build("t3", cust=("region", 1), supp=("region", c % 5),
+                                           date=("year_range", 1992, 1997), group="nation")))
+        e = next(r for r in p["rels"] if r["relOp"] == "PROJECT")["exprs"][-1]
+        e.update(input=c, name="$%d" % c)
+        plans.append(p)
+    want = [PO.execute_plan(p, tables).rows() for p in plans]
+    with Engine() as eng:
+        eng.load_tables(tables)
+        for some in (plans, plans[2:5], plans):
+            got, batched = eng.execute_batch(some)
+            assert batched == len(some)
+            assert [g.rows() for g in got] == [want[plans.index(p)] for p in some]
