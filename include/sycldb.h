@@ -519,11 +519,13 @@ uint64_t sdb_result_selected(const sdb_result *r);
 int sdb_result_selected_rows(const sdb_result *r, uint64_t *host);
 int sdb_result_col_copy_selected(const sdb_result *r, int c, void *host);
 /* The same in two calls: what a result holds, and its selected rows in one
- * buffer of selected_bytes bytes: the row numbers (uint64), then each column's
- * values (int32 or uint64) from the next multiple of 8 bytes on.  Bit c of
- * u64_cols: column c (below 64) holds uint64 sums. */
+ * buffer: the row numbers (uint64), then each column's values (int32 or
+ * uint64) from the next multiple of 8 bytes on.  selected is UINT64_MAX where
+ * counting takes a pass over the flags (sdb_result_selected does that: a table
+ * of 32,768 rows or more that is no group-by result).  Bit c of u64_cols:
+ * column c (below 64) holds uint64 sums. */
 typedef struct sdb_result_info {
-    uint64_t nrows, selected, selected_bytes, u64_cols;
+    uint64_t nrows, selected, u64_cols;
     int ncols;
 } sdb_result_info;
 int sdb_result_describe(const sdb_result *r, sdb_result_info *info);

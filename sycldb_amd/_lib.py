@@ -84,7 +84,6 @@ class RequestInfo(ctypes.Structure):
 class ResultInfo(ctypes.Structure):
     _fields_ = [("nrows", ctypes.c_uint64),
                 ("selected", ctypes.c_uint64),
-                ("selected_bytes", ctypes.c_uint64),
                 ("u64_cols", ctypes.c_uint64),
                 ("ncols", ctypes.c_int)]
 

@@ -495,7 +495,6 @@ struct ResultTable {
     void col_selected_to(int c, void *host) const;      // selected() values
     void list_selected();                               // fills sel of a dense table
     // row ids (uint64), then every column's values, each part 8-byte aligned
-    uint64_t selected_bytes() const;
     void selected_to(uint8_t *host) const;
 };
 

@@ -730,8 +730,9 @@ int sdb_result_describe(const sdb_result *r, sdb_result_info *info)
     return guarded([&] {
         require(r && info, "null argument");
         info->nrows = r->t.nrows;
-        info->selected = r->t.selected();
-        info->selected_bytes = r->t.selected_bytes();
+        // (an unlisted table's rows are counted by a pass over its flags, when
+        // the caller asks for them)
+        info->selected = r->t.sparse || r->t.listed ? r->t.selected() : UINT64_MAX;
         info->ncols = (int)r->t.cols.size();
         info->u64_cols = 0;
         for (size_t c = 0; c < r->t.cols.size() && c < 64; c++)

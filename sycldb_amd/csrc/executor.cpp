@@ -556,14 +556,6 @@ void ResultTable::list_selected()
     listed = true;
 }
 
-uint64_t ResultTable::selected_bytes() const
-{
-    const uint64_t k = selected();
-    uint64_t b = 8 * k;
-    for (const Col &c : cols) b += ((c.is_u64 ? 8 : 4) * k + 7) / 8 * 8;
-    return b;
-}
-
 void ResultTable::selected_to(uint8_t *host) const
 {
     const uint64_t k = selected();

@@ -46,14 +46,17 @@ class Result:
         if self._selected is None:
             # one call for the row numbers and every column's values
             k = self._info.selected
-            buf = np.empty(self._info.selected_bytes, np.uint8)
+            if k == 2**64 - 1:  # not counted yet
+                k = int(L.lib.sdb_result_selected(self._h))
+            kinds = self._u64()
+            buf = np.empty(8 * k + sum((8 if u64 else 4) * k + 7 & ~7 for u64 in kinds), np.uint8)
             if k:
                 L.check(L.lib.sdb_result_selected_copy(self._h, buf.ctypes.data))
             at, cols = 8 * k, []
-            for u64 in self._u64():
+            for u64 in kinds:
                 end = at + (8 if u64 else 4) * k
                 cols.append(buf[at:end].view(np.uint64 if u64 else np.int32))
-                at = (end + 7) // 8 * 8
+                at = end + 7 & ~7
             self._selected = (buf[:8 * k].view(np.uint64), cols)
         return self._selected
 
