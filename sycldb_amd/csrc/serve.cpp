@@ -93,9 +93,10 @@ uint64_t estimate_footprint(Engine &eng, const PlanResult &plan)
 // program in a shared scan, as a fraction of its plain run (measured at 600M
 // rows: 0.4-0.9 ms per extra program against 1.6-2.7 ms alone), and the
 // fixed part assumed before any batch has run on an engine, in plain runs
-// (measured at 600M rows: ~6 ms against 1.6 ms alone).
+// (with that marginal cost, batches of 8: 2.1 over 200,000 rows; over 600M
+// rows 1.8 for q1.x and q4.x, 2.4 for q3.x, 5 for q2.x).
 constexpr double BATCH_MARGINAL = 0.3;
-constexpr double BATCH_FIXED_INITIAL = 4.0;
+constexpr double BATCH_FIXED_INITIAL = 2.0;
 // Wave slots per CU (of 32) a batched scan may take while other engines'
 // workers run: a batched kernel that fills every slot makes the others'
 // kernels wait for its whole scan.
