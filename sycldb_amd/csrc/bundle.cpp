@@ -61,8 +61,8 @@ static void dump_program(const FProgram &p, int64_t n, const std::string &table)
         return e && *e && *e != '0';
     }();
     if (!on) return;
-    fprintf(stderr, "[fused %s] rows=%lld vec=%d instr=%d vals=%d prefetch=%d blobs=%d lds=%u group=%d\n",
-            table.c_str(), (long long)n, p.vec, p.ninstr, p.nvals, p.npf, p.nblobs, p.lds_bytes, p.gb.lds);
+    fprintf(stderr, "[fused %s] rows=%lld vec=%d instr=%d vals=%d prefetch=%d blobs=%d lds=%u group=%d fold=%u\n",
+            table.c_str(), (long long)n, p.vec, p.ninstr, p.nvals, p.npf, p.nblobs, p.lds_bytes, p.gb.lds, p.fold);
     for (int i = 0; i < p.ninstr; i++) {
         const FInstr &I = p.ins[i];
         fprintf(stderr, "  %2d %-12s in=%d out=%d logic=%d va=%d vb=%d vout=%d lds=%d vkind=%d store=%d\n", i,

@@ -485,7 +485,10 @@ struct Gen {
                 c << "            " << fout << " = o;\n        }\n";
                 break;
             }
-            const std::string fin = folded(i) ? fold_reg(i) : freg(I.fin) + "[u]";
+            // a probe issued early read its table for the rows of that time:
+            // those the instructions between have dropped stay dropped
+            const std::string now = freg(I.fin) + "[u]";
+            const std::string fin = !folded(i) ? now : hoisted[i] ? "(" + fold_reg(i) + " & " + now + ")" : fold_reg(i);
             c << U << "{\n            uint32_t o = 0;\n";
             if (!vout || late_value(i)) c << "            int32_t none[R];\n";
             c << "            if (" << fin << ") {\n";

@@ -1,5 +1,9 @@
 """Forms of the fused fact kernels that only large or wide programs take,
 against the same plans run one kernel per operator."""
+import os
+import subprocess
+import sys
+
 import pytest
 
 pytestmark = pytest.mark.gpu
@@ -9,6 +13,7 @@ from sycldb_amd import plans as PL  # noqa: E402
 from sycldb_amd import schema as S  # noqa: E402
 from sycldb_amd.engine import Engine  # noqa: E402
 
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 T2 = (S.LO_PARTKEY, S.LO_SUPPKEY, S.LO_ORDERDATE, S.LO_REVENUE)
 
 
@@ -50,3 +55,40 @@ def test_groupby_forms(cust, supp, codegen):
     with Engine(codegen=codegen) as eng:
         eng.generate(300_007, 45)
         assert eng.execute(plan).rows() == want and len(want) > 100
+
+
+# Run in a process of its own: the switch is read once.
+EARLY = """
+from sycldb_amd import plans as PL, schema as S
+from sycldb_amd.engine import Engine
+cols = (S.LO_QUANTITY, S.LO_CUSTKEY, S.LO_SUPPKEY, S.LO_REVENUE)
+b = PL.PlanBuilder()
+b.scan("lineorder")
+lo = b.filter(PL.expr("<", PL.col(S.LO_QUANTITY), PL.lit(25)))
+b.scan("customer")
+cust = b.filter(PL.expr("=", PL.col(S.C_NATION), PL.lit(6)))
+j1 = b.join(lo, cust, S.LO_CUSTKEY, S.C_CUSTKEY)
+c_at = b.offset(lo) + S.C_NATION
+b.scan("supplier")
+supp = b.filter(PL.search(PL.col(S.S_CITY), PL.closed_range(20, 79)))
+s_at = b.offset(j1) + S.S_NATION
+b.join(j1, supp, S.LO_SUPPKEY, S.S_SUPPKEY)
+b.project([PL.col(c_at), PL.col(s_at), PL.col(S.LO_REVENUE)], ["c_nation", "s_nation", "lo_revenue"])
+b.aggregate([0, 1], 2, "revenue")
+with Engine(codegen="compile") as eng:
+    eng.generate((1 << 25) + 1027, 11, sizes={"customer": 1_400_000}, fact_columns=cols)
+    fused = eng.execute(b.plan()).rows()
+    eng.set_fusion(False)
+    assert fused == eng.execute(b.plan()).rows() and len(fused) > 0
+"""
+
+
+def test_filtered_probe_issued_early():
+    """SDB_JIT_HOIST=1 issues the customer probe's reads, behind their
+    presence filter, with the supplier's value reads: rows that the supplier
+    drops in between stay dropped."""
+    out = subprocess.run([sys.executable, "-c", EARLY], cwd=ROOT, capture_output=True, text=True, timeout=110,
+                         env=dict(os.environ, SDB_JIT_HOIST="1", SDB_DEBUG_FUSED="1"))
+    print(out.stderr[-4000:])
+    assert out.returncode == 0, out.stdout
+    assert "fold=3" in out.stderr  # the filtered probe comes third
