@@ -14,7 +14,10 @@
  *     two's-complement int64 sum;
  *   - `stream` is a hipStream_t (NULL = the default stream); operators are
  *     asynchronous and ordered by the stream, as the reference's kernels are
- *     ordered by event dependencies;
+ *     ordered by event dependencies.  Operators that need scratch memory keep
+ *     a buffer per stream, so calls on different streams and from several
+ *     threads may overlap; graphs captured on one stream share one, so their
+ *     replays may not overlap each other;
  *   - lengths are int64 (the reference's `int col_len` is at most 2^28);
  *   - the return value is a status: SDB_OK, or an SDB_ERR_* code whose text
  *     sdb_last_error() returns (per thread).  No C++ exception crosses the

@@ -144,7 +144,10 @@ void sdb_engine_destroy(sdb_engine *e)
     if (eng.sync_ev) (void)hipEventDestroy(eng.sync_ev);
     if (eng.ev_start) (void)hipEventDestroy(eng.ev_start);
     if (eng.ev_stop) (void)hipEventDestroy(eng.ev_stop);
-    if (eng.stream) (void)hipStreamDestroy(eng.stream);
+    if (eng.stream) {
+        scratch_release(eng.stream);
+        (void)hipStreamDestroy(eng.stream);
+    }
     delete e;
 }
 

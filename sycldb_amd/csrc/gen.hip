@@ -7,7 +7,10 @@
 // a table of any size is produced in one pass at HBM write speed.
 #include "capi_util.hpp"
 
+#include <atomic>
+#include <map>
 #include <mutex>
+#include <tuple>
 #include <vector>
 
 namespace sdb {
@@ -63,12 +66,7 @@ __global__ void __launch_bounds__(BLOCK) k_gen_rowid(int32_t *out, int64_t n, in
 
 thread_local std::string g_last_error;
 
-struct Scratch {
-    void *ptr = nullptr;
-    size_t bytes = 0;
-};
-std::mutex g_scratch_mu;
-std::vector<Scratch> g_scratch;   // per device
+std::mutex g_cu_mu;
 std::vector<int> g_cu_count;      // per device, 0 = unknown
 
 } // namespace
@@ -79,7 +77,7 @@ int device_cu_count()
 {
     int dev = 0;
     SDB_HIP(hipGetDevice(&dev));
-    std::lock_guard<std::mutex> lk(g_scratch_mu);
+    std::lock_guard<std::mutex> lk(g_cu_mu);
     if ((int)g_cu_count.size() <= dev) g_cu_count.resize(dev + 1, 0);
     if (g_cu_count[dev] == 0) {
         int cus = 0;
@@ -97,25 +95,182 @@ unsigned stream_grid(int64_t units, int64_t per_block, int blocks_per_cu)
     return (unsigned)std::max<int64_t>(1, std::min(need, cap));
 }
 
-void *scratch_buffer(size_t bytes, hipStream_t stream)
-{
-    int dev = 0;
-    SDB_HIP(hipGetDevice(&dev));
-    std::lock_guard<std::mutex> lk(g_scratch_mu);
-    if ((int)g_scratch.size() <= dev) g_scratch.resize(dev + 1);
-    Scratch &s = g_scratch[dev];
-    if (s.bytes < bytes) {
-        if (s.ptr) {
-            SDB_HIP(hipStreamSynchronize(stream));
-            SDB_HIP(hipFree(s.ptr));
-            s.ptr = nullptr;
-            s.bytes = 0;
-        }
-        size_t want = std::max<size_t>(bytes, 1 << 20);
-        SDB_HIP(hipMalloc(&s.ptr, want));
-        s.bytes = want;
+// ------------------------------------------------------------------ scratch
+
+struct ScratchBuffer {
+    std::mutex mu;   // held by the call that uses the buffer
+    void *ptr = nullptr;
+    size_t bytes = 0;
+    uint64_t used = 0;     // when last asked for (under the pool's mutex)
+    bool dropped = false;  // no longer in the pool (under both)
+};
+
+namespace {
+
+// What a buffer belongs to.  A stream's handle names it: a destroyed stream's
+// handle may come back for a new one, but only after its work is done
+// (hipStreamDestroy waits for it).  hipStreamPerThread is one handle for every
+// thread's own stream.
+struct ScratchKey {
+    int dev;
+    hipStream_t stream;
+    uint64_t thread; // 0 but for hipStreamPerThread
+    bool captured;
+    bool operator<(const ScratchKey &o) const
+    {
+        return std::tie(dev, stream, thread, captured) < std::tie(o.dev, o.stream, o.thread, o.captured);
     }
-    return s.ptr;
+};
+
+// At most SCRATCH_MAX_BUFFERS per device outside captures, and past
+// SCRATCH_MAX_BYTES in all only the one in use: the longest unused go first.
+constexpr size_t SCRATCH_MAX_BUFFERS = 32;
+constexpr size_t SCRATCH_MAX_BYTES = size_t(1) << 30;
+struct ScratchPool {
+    std::mutex mu;
+    std::map<ScratchKey, std::shared_ptr<ScratchBuffer>> buffers;
+    uint64_t clock = 0;
+};
+// (never destroyed: the runtime may be gone before this library's statics)
+ScratchPool &scratch_pool()
+{
+    static ScratchPool *p = new ScratchPool;
+    return *p;
+}
+
+uint64_t thread_number()
+{
+    static std::atomic<uint64_t> next{1};
+    thread_local const uint64_t n = next++;
+    return n;
+}
+
+ScratchKey scratch_key(hipStream_t stream)
+{
+    ScratchKey k{0, stream, stream == hipStreamPerThread ? thread_number() : 0, false};
+    SDB_HIP(hipGetDevice(&k.dev));
+    if (stream) {
+        hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+        if (hipStreamIsCapturing(stream, &st) == hipSuccess) k.captured = st == hipStreamCaptureStatusActive;
+        else (void)hipGetLastError(); // a stream that cannot be captured now
+    }
+    return k;
+}
+
+// While a stream is captured, allocations are refused unless the thread says
+// that it means them.
+struct RelaxedCapture {
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    RelaxedCapture() { SDB_HIP(hipThreadExchangeStreamCaptureMode(&mode)); }
+    ~RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+};
+
+// Drops buffers of the device (never `keep`, one in use or one of a capture)
+// until `bytes` more stay within the pool's bounds.  hipFree waits for the
+// device, so for the kernels that still use one.
+void scratch_trim(ScratchPool &P, const ScratchKey &key, const ScratchBuffer *keep, size_t bytes)
+{
+    while (true) {
+        size_t count = 0, total = bytes;
+        auto oldest = P.buffers.end();
+        for (auto it = P.buffers.begin(); it != P.buffers.end(); ++it) {
+            if (it->first.dev != key.dev || it->first.captured) continue;
+            count++;
+            if (it->second.get() == keep) continue;
+            total += it->second->bytes;
+            if (it->second->mu.try_lock()) {
+                if (oldest == P.buffers.end() || it->second->used < oldest->second->used) {
+                    if (oldest != P.buffers.end()) oldest->second->mu.unlock();
+                    oldest = it;
+                } else {
+                    it->second->mu.unlock();
+                }
+            }
+        }
+        if (oldest == P.buffers.end()) return;
+        const std::shared_ptr<ScratchBuffer> b = oldest->second;
+        const bool drop = count > SCRATCH_MAX_BUFFERS || total > SCRATCH_MAX_BYTES;
+        if (drop) {
+            b->dropped = true;
+            P.buffers.erase(oldest);
+            if (b->ptr) (void)hipFree(b->ptr);
+            b->ptr = nullptr;
+            b->bytes = 0;
+        }
+        b->mu.unlock();
+        if (!drop) return;
+    }
+}
+
+} // namespace
+
+Scratch::Scratch(size_t bytes, hipStream_t stream)
+{
+    const ScratchKey key = scratch_key(stream);
+    ScratchPool &P = scratch_pool();
+    while (true) {
+        {
+            std::lock_guard<std::mutex> lk(P.mu);
+            std::shared_ptr<ScratchBuffer> &b = P.buffers[key];
+            if (!b) b = std::make_shared<ScratchBuffer>();
+            b->used = ++P.clock;
+            buf_ = b;
+        }
+        buf_->mu.lock();
+        if (!buf_->dropped) break;
+        buf_->mu.unlock();
+    }
+    if (buf_->bytes >= bytes) return;
+    try {
+        const size_t want = std::max<size_t>(bytes, 1 << 20);
+        RelaxedCapture relaxed;
+        std::lock_guard<std::mutex> lk(P.mu);
+        if (!key.captured) {
+            if (buf_->ptr) {
+                SDB_HIP(hipStreamSynchronize(stream));
+                SDB_HIP(hipFree(buf_->ptr));
+            }
+            buf_->ptr = nullptr;
+            buf_->bytes = 0;
+            scratch_trim(P, key, buf_.get(), want);
+        }
+        // (a captured buffer that has become too small stays for its graphs;
+        // each new one is twice as large at least, so they add up to little)
+        const size_t size = key.captured ? std::max(want, 2 * buf_->bytes) : want;
+        void *p = nullptr;
+        SDB_HIP(hipMalloc(&p, size));
+        buf_->ptr = p;
+        buf_->bytes = size;
+    } catch (...) {
+        buf_->mu.unlock();
+        throw;
+    }
+}
+
+Scratch::~Scratch() { buf_->mu.unlock(); }
+
+uint8_t *Scratch::data() const { return static_cast<uint8_t *>(buf_->ptr); }
+
+void scratch_release(hipStream_t stream)
+{
+    ScratchKey key{0, stream, 0, false};
+    if (hipGetDevice(&key.dev) != hipSuccess) return;
+    ScratchPool &P = scratch_pool();
+    std::shared_ptr<ScratchBuffer> b;
+    {
+        std::lock_guard<std::mutex> lk(P.mu);
+        auto it = P.buffers.find(key);
+        if (it == P.buffers.end()) return;
+        b = it->second;
+    }
+    std::lock_guard<std::mutex> own(b->mu); // (before the pool's, as a call that grows its buffer)
+    std::lock_guard<std::mutex> lk(P.mu);
+    if (b->dropped) return;
+    b->dropped = true;
+    P.buffers.erase(key);
+    if (b->ptr) (void)hipFree(b->ptr);
+    b->ptr = nullptr;
+    b->bytes = 0;
 }
 
 } // namespace sdb

@@ -2119,7 +2119,8 @@ void launch_probe_full(const int32_t *probe, int32_t *val_out, const uint8_t *in
     if (n >= PROBE_U16_MIN_ROWS && len > 0 && len * PROBE_U16_MIN_RATIO <= n && len <= PROBE_U16_MAX_SLOTS) {
         const size_t words = (size_t)((len + 31) / 32), part_off = 256;
         const size_t u16_off = part_off + PAIRS_RANGE_BLOCKS * 8, bits_off = u16_off + ((size_t)len * 2 + 15) / 16 * 16;
-        uint8_t *scr = static_cast<uint8_t *>(scratch_buffer(bits_off + words * 4, s));
+        const Scratch scratch(bits_off + words * 4, s);
+        uint8_t *scr = scratch.data();
         int32_t *info = reinterpret_cast<int32_t *>(scr);
         int32_t *partials = reinterpret_cast<int32_t *>(scr + part_off);
         uint16_t *u16 = reinterpret_cast<uint16_t *>(scr + u16_off);
@@ -2344,8 +2345,8 @@ int64_t compact_tiles(int64_t n) { return n > 0 ? (n + COMPACT_TILE - 1) / COMPA
 void launch_compact(const uint8_t *flags, int64_t n, int32_t *row_ids, uint32_t *count, hipStream_t s)
 {
     const int64_t ntiles = compact_tiles(n);
-    uint32_t *counts = reinterpret_cast<uint32_t *>(scratch_buffer((size_t)std::max<int64_t>(ntiles, 1) * 4, s));
-    launch_compact_into(flags, n, row_ids, count, counts, s);
+    const Scratch scratch((size_t)std::max<int64_t>(ntiles, 1) * 4, s);
+    launch_compact_into(flags, n, row_ids, count, reinterpret_cast<uint32_t *>(scratch.data()), s);
 }
 
 void launch_compact_into(const uint8_t *flags, int64_t n, int32_t *row_ids, uint32_t *count, uint32_t *counts,
@@ -2470,7 +2471,8 @@ void launch_gather_i32(const int32_t *src, const int32_t *ids, int64_t count, in
 void minmax_i32(const int32_t *col, int64_t n, int32_t *mn, int32_t *mx, hipStream_t s)
 {
     if (n <= 0) fail(SDB_ERR_INVALID_ARG, "min/max of an empty column");
-    int32_t *mm = reinterpret_cast<int32_t *>(scratch_buffer(8, s));
+    const Scratch scratch(8, s);
+    int32_t *mm = reinterpret_cast<int32_t *>(scratch.data());
     hipLaunchKernelGGL(k_minmax_init, dim3(1), dim3(1), 0, s, mm);
     hipLaunchKernelGGL(k_minmax, dim3(grid_one(n)), dim3(BLOCK), 0, s, col, n, mm);
     check_launch("minmax");
@@ -2730,7 +2732,8 @@ int sdb_compress_sync(const int32_t *const *cols, int ncols, const uint8_t *flag
         // models/transient_table.hpp:535-599, here in row order) ...
         const int64_t ntiles = compact_tiles(n);
         const size_t ids_bytes = ((size_t)n * 4 + 255) / 256 * 256, cnt_off = ids_bytes + (size_t)ntiles * 4;
-        uint8_t *scr = static_cast<uint8_t *>(scratch_buffer(cnt_off + 256, s));
+        const Scratch scratch(cnt_off + 256, s);
+        uint8_t *scr = scratch.data();
         int32_t *ids = reinterpret_cast<int32_t *>(scr);
         uint32_t *dcount = reinterpret_cast<uint32_t *>(scr + cnt_off);
         launch_compact_into(flags, n, ids, dcount, reinterpret_cast<uint32_t *>(scr + ids_bytes), s);

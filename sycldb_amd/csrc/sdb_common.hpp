@@ -6,6 +6,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <memory>
 #include <stdexcept>
 #include <string>
 
@@ -37,9 +38,28 @@ int device_cu_count();
 // `per_block` items consumed per block iteration.
 unsigned stream_grid(int64_t units, int64_t per_block, int blocks_per_cu = 8);
 
-// Library-owned scratch: a device buffer of at least `bytes`, reused across
-// calls on the same device and stream-ordered by the caller's stream.
-void *scratch_buffer(size_t bytes, hipStream_t stream);
+// Library-owned scratch: a device buffer of at least `bytes` for the calls of
+// one stream.  Work of a stream runs in order, so a call's kernels are done
+// with the buffer before the next call's overwrite it; calls on different
+// streams get different buffers.  Held while the kernels that use it are
+// queued, so that two threads on one stream do not mix theirs.  A call that is
+// being captured gets a buffer of its stream's captures, which is never freed
+// or moved: the graph keeps its address.  (Graphs captured on one stream share
+// it: their replays must not overlap.)
+struct ScratchBuffer;
+class Scratch {
+  public:
+    Scratch(size_t bytes, hipStream_t stream);
+    ~Scratch();
+    Scratch(const Scratch &) = delete;
+    Scratch &operator=(const Scratch &) = delete;
+    uint8_t *data() const;
+
+  private:
+    std::shared_ptr<ScratchBuffer> buf_;
+};
+// Gives back the buffer of a stream about to be destroyed (its work done).
+void scratch_release(hipStream_t stream);
 
 // ------------------------------------------------------- result transfer
 
