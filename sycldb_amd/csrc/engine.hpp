@@ -127,6 +127,7 @@ struct Table {
     uint64_t nrows = 0;
     std::vector<Column> columns;            // table_column_numbers entries
     std::vector<void *> owned;              // device buffers to free
+    ~Table() { forget_batches(this); }
 };
 
 // ------------------------------------------------------------ kernel bundles

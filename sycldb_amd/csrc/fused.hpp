@@ -80,6 +80,8 @@ typedef void *(*BatchAlloc)(void *ctx, size_t bytes);
 // launch shape whose launch is a replayed hipGraph.
 void launch_fused_batch(const std::vector<FProgram> &in, int64_t n, hipStream_t s, int unroll,
                         const void *scope, BatchAlloc alloc, void *alloc_ctx, bool masks = true);
+// The fact table `scope` is gone: its batches' library starts over.
+void forget_batches(const void *scope);
 // Batched launches as replayed hipGraphs (1), as plain stream operations
 // (0), or as SDB_BATCH_GRAPH says (-1, the default: off).
 void set_batch_graphs(int on);

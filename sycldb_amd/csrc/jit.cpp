@@ -2828,33 +2828,6 @@ void order_masks(BatchPlan &b, const std::vector<FProgram> &q, const std::vector
     b.lazy = mode == 1 || (mode < 0 && reads <= 0.75 * nm);
 }
 
-// A library that cannot take this batch's columns beside those met before
-// (a table that took the place of a released one brings new ones) starts over
-// with the batch's own.  Plans made before keep their copies of its state.
-void make_room(BatchLibrary &lib, const std::vector<FProgram> &q)
-{
-    std::vector<const int32_t *> cols = lib.slots;
-    auto add = [&](const int32_t *c) {
-        if (c && std::find(cols.begin(), cols.end(), c) == cols.end()) cols.push_back(c);
-    };
-    for (const FProgram &p : q) {
-        for (int j = 0; j < p.npf; j++) add(p.pf_mem[j]);
-        for (int i = 0; i < p.ninstr; i++) {
-            if (p.ins[i].va < 0) add(p.ins[i].a);
-            if (p.ins[i].vb < 0) add(p.ins[i].b);
-        }
-        for (int j = 0; j < p.gb.k; j++)
-            if (p.gb.key_reg[j] < 0) add(p.gb.key_mem[j]);
-        if (p.gb.k && p.gb.agg_reg < 0) add(p.gb.agg_mem);
-    }
-    if ((int)cols.size() <= BATCH_MAX_PF || lib.slots.empty()) return;
-    lib.slots.clear();
-    lib.mask_slots.clear();
-    lib.bodies.clear();
-    lib.body_of.clear();
-    for (auto &s : lib.srcs) s.second.state[0] = ~size_t(0);
-}
-
 BatchPlan plan_batch(const std::vector<FProgram> &in, int unroll, const std::string &lib_key, bool masks,
                      const BatchShape &shape)
 {
@@ -2866,7 +2839,6 @@ BatchPlan plan_batch(const std::vector<FProgram> &in, int unroll, const std::str
     BatchLibrary &lib = g_libs[lib_key + (b.vec ? "/vec" : "/row") + "/u" + std::to_string(unroll)];
     std::vector<int> shape_of(q.size());
     std::vector<std::vector<int>> shared(q.size());
-    make_room(lib, q);
     for (size_t i = 0; i < q.size(); i++) {
         remap_prefetch(q[i], lib.slots);
         if (masks) shared[i] = shared_probes(q[i]);
@@ -3054,6 +3026,25 @@ BatchPlan plan_batch(const std::vector<FProgram> &in, int unroll, const std::str
 }
 
 } // namespace
+
+// The libraries of a table that is gone start over: their slots name its
+// columns, and a table made later may get its address.
+void forget_batches(const void *scope)
+{
+    char part[40];
+    snprintf(part, sizeof(part), "/%p/", scope);
+    std::lock_guard<std::mutex> lk(g_lib_mu);
+    for (auto &kv : g_libs) {
+        if (kv.first.find(part) == std::string::npos) continue;
+        BatchLibrary &lib = kv.second;
+        lib.slots.clear();
+        lib.mask_slots.clear();
+        lib.bodies.clear();
+        lib.body_of.clear();
+        // (plans keep pointers to the sources: they stay, to be written anew)
+        for (auto &s : lib.srcs) s.second.state[0] = ~size_t(0);
+    }
+}
 
 int jit_batch_check(const std::string &arch)
 {

@@ -121,3 +121,57 @@ def test_batch_reads_more_columns_than_the_shared_scan_holds():
             got, batched = eng.execute_batch(some)
             assert batched == len(some)
             assert [g.rows() for g in got] == [want[plans.index(p)] for p in some]
+
+
+def _sum_plans(which):
+    """q3.x sums, each over one of the 17 fact columns."""
+    import json
+    out = []
+    for c in which:
+        p = json.loads(PL.to_json(PL.build("t3", cust=("region", 1), supp=("region", c % 5),
+                                           date=("year_range", 1992, 1997), group="nation")))
+        e = next(r for r in p["rels"] if r["relOp"] == "PROJECT")["exprs"][-1]
+        e.update(input=c, name="$%d" % c)
+        out.append(p)
+    return out
+
+
+def _fact_tables(rows, seed):
+    import numpy as np
+    tables = datagen.generate_tables(S, rows, seed)
+    rng = np.random.default_rng(seed)
+    for c in set(range(17)) - set(tables["lineorder"]):
+        tables["lineorder"][c] = rng.integers(-1000, 1000, rows).astype(np.int32)
+    return tables
+
+
+def test_batches_past_the_shared_scan_keep_their_kernels():
+    """A batch over all 17 fact columns between others: what the table's
+    batches compiled stays in use, whichever ran last."""
+    from sycldb_amd import engine as E
+    tables = _fact_tables(50_003, 45)
+    one = _sum_plans(range(17))
+    two, three = [PL.build("t1"), PL.build("t4")], [PL.build("t2"), PL.build("t2", s_region=3)]
+    with E.Engine() as eng:
+        eng.load_tables(tables)
+        for some in (one, two, one, three):
+            eng.execute_batch(some)
+        assert E.codegen_wait(100)
+        before = E.codegen_kernels_compiled()
+        for some in (one, two, three):
+            assert eng.execute_batch(some)[1] == len(some)
+        assert E.codegen_wait(100) and E.codegen_kernels_compiled() == before
+
+
+def test_batches_over_a_table_loaded_again():
+    """The fact table replaced (its columns then lie elsewhere, the table
+    itself maybe where it was): the batch's results are the new table's."""
+    from sycldb_amd.engine import Engine
+    plans = _sum_plans(range(4, 16))
+    with Engine() as eng:
+        for seed in (45, 46, 47):
+            tables = _fact_tables(30_001 + seed, seed)
+            eng.load_tables(tables)
+            got, batched = eng.execute_batch(plans)
+            assert batched == len(plans)
+            assert [g.rows() for g in got] == [PO.execute_plan(p, tables).rows() for p in plans]
