@@ -291,23 +291,14 @@ __device__ __forceinline__ int64_t wt_row(int64_t t0, int lane, int j) { return 
 // offset in its tile of the row of mask bit b
 __device__ __forceinline__ uint32_t wt_offset(int lane, uint32_t b) { return (b >> 2) * 256u + 4u * lane + (b & 3u); }
 
-// Flags of a tile (rows at or past n: 0).  VEC: flags 4-byte aligned.
-template <bool VEC>
-__device__ __forceinline__ void wt_flags(const uint8_t *flags, int64_t n, int64_t t0, int lane, uint32_t (&f)[WT_CHUNKS])
+// Flags of a whole tile, at any alignment (global memory takes wide loads at
+// any byte).  The rows past the last whole tile are left to the last block's
+// threads, one each: read here with bounds checks they cost a round trip per
+// row slot, and the registers that a second block per CU needs.
+__device__ __forceinline__ void wt_flags(const uint8_t *flags, int64_t t0, int lane, uint32_t (&f)[WT_CHUNKS])
 {
-    if (VEC && t0 + WT_ROWS <= n) {
 #pragma unroll
-        for (int j = 0; j < WT_CHUNKS; j++) f[j] = *reinterpret_cast<const uint32_t *>(flags + wt_row(t0, lane, j));
-        return;
-    }
-#pragma unroll
-    for (int j = 0; j < WT_CHUNKS; j++) {
-        const int64_t r = wt_row(t0, lane, j);
-        f[j] = 0;
-#pragma unroll
-        for (int k = 0; k < 4; k++)
-            if (r + k < n) f[j] |= (uint32_t)flags[r + k] << (8 * k);
-    }
+    for (int j = 0; j < WT_CHUNKS; j++) __builtin_memcpy(&f[j], flags + wt_row(t0, lane, j), 4);
 }
 
 // Bit k: whether byte k of x is nonzero (the flag bits 0, 8, 16, 24 of
@@ -745,10 +736,10 @@ __global__ void __launch_bounds__(PROBE_BLOCK) k_probe_full_lds(const int32_t *_
     // the wave's row masks and list, behind the filter
     uint32_t *const hit_of = reinterpret_cast<uint32_t *>(probe_lds) + fwords + wave * (64 + cap);
     uint32_t *const list = hit_of + 64;
-    const int64_t ntiles = (n + WT_ROWS - 1) / WT_ROWS, stride = (int64_t)gridDim.x * (PROBE_BLOCK / 64);
+    const int64_t ntiles = n / WT_ROWS, stride = (int64_t)gridDim.x * (PROBE_BLOCK / 64);
     int64_t tile = (int64_t)blockIdx.x * (PROBE_BLOCK / 64) + wave;
     uint32_t next[WT_CHUNKS];
-    if (tile < ntiles) wt_flags<true>(in, n, tile * WT_ROWS, lane, next);
+    if (tile < ntiles) wt_flags(in, tile * WT_ROWS, lane, next);
     for (; tile < ntiles; tile += stride) {
         const int64_t t0 = tile * WT_ROWS;
         const uint32_t flagged = wt_mask(next);
@@ -756,27 +747,18 @@ __global__ void __launch_bounds__(PROBE_BLOCK) k_probe_full_lds(const int32_t *_
 #pragma unroll
         for (int j = 0; j < WT_CHUNKS; j++) other |= next[j] & 0xfefefefeu;
         const bool odd = other != 0;
-        const bool whole = t0 + WT_ROWS <= n;
         uint32_t slot[WT_CHUNKS][4];
 #pragma unroll
         for (int j = 0; j < WT_CHUNKS; j++) {
-            const int64_t r = wt_row(t0, lane, j);
             int4 x = make_int4(0, 0, 0, 0);
-            if ((flagged >> (4 * j)) & 15u) {
-                if (whole || r + 3 < n) x = *reinterpret_cast<const int4 *>(probe + r);
-                else {
-                    x.x = probe[r];
-                    if (r + 1 < n) x.y = probe[r + 1];
-                    if (r + 2 < n) x.z = probe[r + 2];
-                }
-            }
+            if ((flagged >> (4 * j)) & 15u) x = *reinterpret_cast<const int4 *>(probe + wt_row(t0, lane, j));
             slot[j][0] = (uint32_t)x.x - (uint32_t)min;
             slot[j][1] = (uint32_t)x.y - (uint32_t)min;
             slot[j][2] = (uint32_t)x.z - (uint32_t)min;
             slot[j][3] = (uint32_t)x.w - (uint32_t)min;
         }
         // the next tile's flags load while this one is probed
-        if (tile + stride < ntiles) wt_flags<true>(in, n, t0 + stride * WT_ROWS, lane, next);
+        if (tile + stride < ntiles) wt_flags(in, t0 + stride * WT_ROWS, lane, next);
         uint32_t cand = 0;
 #pragma unroll
         for (int b = 0; b < 4 * WT_CHUNKS; b++) {
@@ -863,12 +845,28 @@ __global__ void __launch_bounds__(PROBE_BLOCK) k_probe_full_lds(const int32_t *_
             const uint32_t f = flag_bytes(hits >> (4 * j));
             // in place, flags that stay as they are need no write
             if (in == out && !__any(odd || (((hits ^ flagged) >> (4 * j)) & 15u))) continue;
-            if (whole || r + 3 < n) *reinterpret_cast<uint32_t *>(out + r) = f;
-            else
-                for (int k = 0; k < 4; k++)
-                    if (r + k < n) out[r + k] = (uint8_t)(f >> (8 * k));
+            *reinterpret_cast<uint32_t *>(out + r) = f;
         }
     }
+    if (blockIdx.x + 1 == gridDim.x)
+        for (int64_t i = ntiles * WT_ROWS + threadIdx.x; i < n; i += PROBE_BLOCK) {
+            const uint32_t s = (uint32_t)probe[i] - (uint32_t)min;
+            bool hit = false;
+            if (in[i] && s <= span) {
+                int32_t v;
+                if (use16) {
+                    const uint32_t raw = VALS ? reinterpret_cast<const uint16_t *>(probe_lds)[s] : t.u16[s];
+                    v = vmin + (int32_t)raw;
+                    hit = raw != VALS_UNSET;
+                } else {
+                    const int2 e = t.pairs[s];
+                    v = e.y;
+                    hit = e.x == 1;
+                }
+                if (hit) val_out[i] = v;
+            }
+            out[i] = hit;
+        }
 }
 
 // ----------------------------------------------------------- aggregation
@@ -944,31 +942,26 @@ __global__ void __launch_bounds__(RED_BLOCK) k_sum_flagged(const int32_t *__rest
     block_add_u64((uint64_t)s, acc);
 }
 
-// vec: 16 flags per load (16-byte aligned), else one
-__global__ void __launch_bounds__(RED_BLOCK) k_count_flags(const uint8_t *flags, int64_t n, uint64_t *acc, int vec)
+// 16 flags per load, at any alignment (200M flags 4 bytes past an aligned start:
+// 130 us one by one, 63 four at a time where aligned to 4, 35 so).
+__global__ void __launch_bounds__(RED_BLOCK) k_count_flags(const uint8_t *flags, int64_t n, uint64_t *acc)
 {
     uint64_t s = 0;
-    if (vec) {
-        const int64_t nq = n >> 4;
-        const uint4 *f4 = reinterpret_cast<const uint4 *>(flags);
-        for (int64_t base = (int64_t)blockIdx.x * RED_BLOCK * UNROLL; base < nq;
-             base += (int64_t)gridDim.x * RED_BLOCK * UNROLL) {
-            uint4 q[UNROLL];
+    const int64_t nq = n >> 4;
+    for (int64_t base = (int64_t)blockIdx.x * RED_BLOCK * UNROLL; base < nq;
+         base += (int64_t)gridDim.x * RED_BLOCK * UNROLL) {
+        uint4 q[UNROLL];
 #pragma unroll
-            for (int u = 0; u < UNROLL; u++) {
-                const int64_t c = base + u * RED_BLOCK + threadIdx.x;
-                q[u] = c < nq ? f4[c] : make_uint4(0, 0, 0, 0);
-            }
-#pragma unroll
-            for (int u = 0; u < UNROLL; u++)
-                s += __popc(nz_bytes(q[u].x)) + __popc(nz_bytes(q[u].y)) + __popc(nz_bytes(q[u].z)) +
-                     __popc(nz_bytes(q[u].w));
+        for (int u = 0; u < UNROLL; u++) {
+            const int64_t c = base + u * RED_BLOCK + threadIdx.x;
+            q[u] = make_uint4(0, 0, 0, 0);
+            if (c < nq) __builtin_memcpy(&q[u], flags + 16 * c, 16);
         }
-        if (blockIdx.x == 0 && threadIdx.x < (n & 15)) s += flags[(nq << 4) + threadIdx.x] != 0;
-    } else {
-        for (int64_t i = (int64_t)blockIdx.x * RED_BLOCK + threadIdx.x; i < n; i += (int64_t)gridDim.x * RED_BLOCK)
-            s += flags[i] != 0;
+#pragma unroll
+        for (int u = 0; u < UNROLL; u++)
+            s += __popc(nz_bytes(q[u].x)) + __popc(nz_bytes(q[u].y)) + __popc(nz_bytes(q[u].z)) + __popc(nz_bytes(q[u].w));
     }
+    if (blockIdx.x == 0 && threadIdx.x < (n & 15)) s += flags[(nq << 4) + threadIdx.x] != 0;
     block_add_u64(s, acc);
 }
 
@@ -1030,13 +1023,14 @@ __global__ void __launch_bounds__(BLOCK) k_groupby_global(GroupArgs g, const int
 // instead (each lane its own rows) costs a round trip to memory per row slot
 // that any lane of the wave has flagged, nearly all of them already at 1 % of
 // the rows (2^28 rows, 0.8 % flagged, 7,000 slots: 736 -> 189 us;
-// 60M rows, 1.6 %, 175 slots: 274 -> 70 us).
+// 60M rows, 1.6 %, 175 slots: 274 -> 70 us; every row flagged, three keys of
+// 4,375 slots: 514 -> 200 us).
 constexpr int GB_BLOCK = 1024; // threads per block of the LDS group-by
 constexpr int GB_DRAIN = 4;
 constexpr uint32_t GB_LIST = 512; // listed rows per wave: two of a dense tile's chunks
 
 // K: number of keys (0: g.k, up to GB_MAX_KEYS)
-template <int K, bool VEC>
+template <int K>
 __global__ void __launch_bounds__(GB_BLOCK) k_groupby_lds(GroupArgs g, const int32_t *agg, const uint8_t *flags,
                                                           int64_t n, uint64_t *sums, uint32_t *seen, uint32_t prod)
 {
@@ -1050,17 +1044,35 @@ __global__ void __launch_bounds__(GB_BLOCK) k_groupby_lds(GroupArgs g, const int
     for (uint32_t s = threadIdx.x; s < prod; s += GB_BLOCK) lsum[s] = 0;
     for (uint32_t w = threadIdx.x; w < nwords; w += GB_BLOCK) lbits[w] = 0;
     __syncthreads();
+    auto take = [&](const int32_t (&kv)[KMAX], int32_t v) {
+        bool in_range = true;
+        uint32_t s = 0, mult = 1;
+#pragma unroll
+        for (int j = 0; j < KMAX; j++)
+            if (j < nk) {
+                in_range &= kv[j] >= g.mins[j] && kv[j] <= g.maxs[j];
+                s += ((uint32_t)kv[j] - (uint32_t)g.mins[j]) * mult;
+                mult *= g.range[j];
+            }
+        if (!in_range) {
+            group_row_global(g, kv, v, sums, seen, prod);
+            return;
+        }
+        // in range, s is below prod (the ranges multiply to it)
+        atomicAdd(&lsum[s], (unsigned long long)(int64_t)v);
+        if (!((lbits[s >> 5] >> (s & 31)) & 1u)) atomicOr(&lbits[s >> 5], 1u << (s & 31));
+    };
     const int lane = threadIdx.x & 63;
     uint16_t *list = lists[threadIdx.x >> 6];
-    const int64_t ntiles = (n + WT_ROWS - 1) / WT_ROWS, stride = (int64_t)gridDim.x * (GB_BLOCK / 64);
+    const int64_t ntiles = n / WT_ROWS, stride = (int64_t)gridDim.x * (GB_BLOCK / 64);
     int64_t t = (int64_t)blockIdx.x * (GB_BLOCK / 64) + (threadIdx.x >> 6);
     uint32_t next[WT_CHUNKS];
-    if (t < ntiles) wt_flags<VEC>(flags, n, t * WT_ROWS, lane, next);
+    if (t < ntiles) wt_flags(flags, t * WT_ROWS, lane, next);
     for (; t < ntiles; t += stride) {
         const int64_t t0 = t * WT_ROWS;
         const uint32_t tile = wt_mask(next);
         // the next tile's flags load while this one's rows are taken
-        if (t + stride < ntiles) wt_flags<VEC>(flags, n, t0 + stride * WT_ROWS, lane, next);
+        if (t + stride < ntiles) wt_flags(flags, t0 + stride * WT_ROWS, lane, next);
         uint32_t total;
         uint32_t at = wave_prefix((uint32_t)__popc(tile), lane, total);
         const int parts = total <= GB_LIST ? 1 : 4;
@@ -1073,42 +1085,36 @@ __global__ void __launch_bounds__(GB_BLOCK) k_groupby_lds(GroupArgs g, const int
             for (; m; m &= m - 1) list[at++] = (uint16_t)wt_offset(lane, (uint32_t)__builtin_ctz(m) + 8u * part);
             wave_sync();
             for (uint32_t e = 0; e < count; e += 64 * GB_DRAIN) {
+                // (lanes past the list read its last row again: loads under
+                // a condition of their own waited for each other)
                 int32_t kv[GB_DRAIN][KMAX], v[GB_DRAIN];
+                uint32_t o[GB_DRAIN];
+#pragma unroll
+                for (int d = 0; d < GB_DRAIN; d++) o[d] = list[min(e + 64 * d + lane, count - 1)];
 #pragma unroll
                 for (int d = 0; d < GB_DRAIN; d++) {
-                    const uint32_t i = e + 64 * d + lane;
-                    if (i < count) {
-                        const int64_t row = t0 + list[i];
-#pragma unroll
-                        for (int j = 0; j < KMAX; j++)
-                            if (j < nk) kv[d][j] = g.keys[j][row];
-                        v[d] = agg[row];
-                    }
-                }
-#pragma unroll
-                for (int d = 0; d < GB_DRAIN; d++) {
-                    if (e + 64 * d + lane >= count) continue;
-                    bool in_range = true;
-                    uint32_t s = 0, mult = 1;
+                    const int64_t row = t0 + o[d];
 #pragma unroll
                     for (int j = 0; j < KMAX; j++)
-                        if (j < nk) {
-                            in_range &= kv[d][j] >= g.mins[j] && kv[d][j] <= g.maxs[j];
-                            s += ((uint32_t)kv[d][j] - (uint32_t)g.mins[j]) * mult;
-                            mult *= g.range[j];
-                        }
-                    if (!in_range) {
-                        group_row_global(g, kv[d], v[d], sums, seen, prod);
-                        continue;
-                    }
-                    // in range, s is below prod (the ranges multiply to it)
-                    atomicAdd(&lsum[s], (unsigned long long)(int64_t)v[d]);
-                    if (!((lbits[s >> 5] >> (s & 31)) & 1u)) atomicOr(&lbits[s >> 5], 1u << (s & 31));
+                        if (j < nk) kv[d][j] = g.keys[j][row];
+                    v[d] = agg[row];
                 }
+#pragma unroll
+                for (int d = 0; d < GB_DRAIN; d++)
+                    if (e + 64 * d + lane < count) take(kv[d], v[d]);
             }
             wave_sync();
         }
     }
+    if (blockIdx.x + 1 == gridDim.x)
+        for (int64_t i = ntiles * WT_ROWS + threadIdx.x; i < n; i += GB_BLOCK) {
+            if (!flags[i]) continue;
+            int32_t kv[KMAX];
+#pragma unroll
+            for (int j = 0; j < KMAX; j++)
+                if (j < nk) kv[j] = g.keys[j][i];
+            take(kv, agg[i]);
+        }
     __syncthreads();
     for (uint32_t s = threadIdx.x; s < prod; s += GB_BLOCK) {
         if (!((lbits[s >> 5] >> (s & 31)) & 1u)) continue;
@@ -1544,10 +1550,12 @@ __global__ void __launch_bounds__(DICT_BLOCK) k_batch_dict(const FMaskDict *dict
 // ------------------------------------------------------------ compaction
 // Three passes over tiles of COMPACT_TILE rows, one wave per tile: count per
 // tile, exclusive scan of the counts (one block), then write ids in row order.
-// Flags come in 16 to a lane and load; a wave never waits for another one in
-// the counting and writing passes (100M rows, one in twenty
-// flagged: count 93 -> 18 us, scan 62 -> 6 us, write 181 -> 37 us; the count
-// streams its flags at 5.7 TB/s).
+// Flags come in 16 to a lane and load, at any alignment; a wave never waits for
+// another one in the counting and writing passes (100M rows, one in twenty
+// flagged: count 93 -> 18 us, scan 62 -> 6 us, write 181 -> 23 us; the count
+// streams its flags at 5.7 TB/s).  A ragged end is read with the flags before
+// it, in one load: byte by byte it cost a round trip each (200,001 rows 24 us,
+// 17 so; 3M rows one byte past an aligned start 24.7 and 16).
 constexpr int COMPACT_STEPS = 4; // steps of 64 lanes x 16 flags per tile
 constexpr int64_t COMPACT_TILE = (int64_t)64 * 16 * COMPACT_STEPS;
 constexpr int COMPACT_WAVES = BLOCK / 64; // tiles per block
@@ -1558,17 +1566,30 @@ __device__ __forceinline__ uint32_t nz_mask(const uint4 &q)
     return nz_mask(q.x) | nz_mask(q.y) << 4 | nz_mask(q.z) << 8 | nz_mask(q.w) << 12;
 }
 
+// Mask of the flags r .. r + 15 (at or past n: 0).
+__device__ __forceinline__ uint32_t flags16(const uint8_t *flags, int64_t n, int64_t r)
+{
+    if (r >= n) return 0;
+    const int64_t a = min(r, n - 16);
+    if (a >= 0) {
+        uint4 q;
+        __builtin_memcpy(&q, flags + a, 16);
+        return nz_mask(q) >> (int)(r - a);
+    }
+    uint32_t m = 0;
+    for (int k = 0; r + k < n; k++) m |= (uint32_t)(flags[r + k] != 0) << k;
+    return m;
+}
+
 // The flags of rows [t0 + 1024 u + 16 lane, ... + 16) as 16-bit masks; rows
-// at or past n are 0.  VEC: flags 16-byte aligned.
-template <bool VEC>
+// at or past n are 0.
 __device__ __forceinline__ void tile_masks(const uint8_t *flags, int64_t n, int64_t t0, int lane,
                                            uint32_t (&m)[COMPACT_STEPS])
 {
-    if (VEC && t0 + COMPACT_TILE <= n) {
+    if (t0 + COMPACT_TILE <= n) {
         uint4 q[COMPACT_STEPS];
 #pragma unroll
-        for (int u = 0; u < COMPACT_STEPS; u++)
-            q[u] = reinterpret_cast<const uint4 *>(flags + t0)[u * 64 + lane];
+        for (int u = 0; u < COMPACT_STEPS; u++) __builtin_memcpy(&q[u], flags + t0 + u * 1024 + lane * 16, 16);
 #pragma unroll
         for (int u = 0; u < COMPACT_STEPS; u++) m[u] = nz_mask(q[u]);
         return;
@@ -1576,13 +1597,10 @@ __device__ __forceinline__ void tile_masks(const uint8_t *flags, int64_t n, int6
 #pragma unroll
     for (int u = 0; u < COMPACT_STEPS; u++) {
         const int64_t r = t0 + u * 1024 + lane * 16;
-        m[u] = 0;
-        for (int k = 0; k < 16; k++)
-            if (r + k < n) m[u] |= (uint32_t)(flags[r + k] != 0) << k;
+        m[u] = flags16(flags, n, r);
     }
 }
 
-template <bool VEC>
 __global__ void __launch_bounds__(BLOCK) k_compact_count(const uint8_t *__restrict__ flags, int64_t n, int64_t ntiles,
                                                          uint32_t *__restrict__ counts)
 {
@@ -1590,7 +1608,7 @@ __global__ void __launch_bounds__(BLOCK) k_compact_count(const uint8_t *__restri
     const int64_t t = (int64_t)blockIdx.x * COMPACT_WAVES + (threadIdx.x >> 6);
     if (t >= ntiles) return;
     uint32_t m[COMPACT_STEPS];
-    tile_masks<VEC>(flags, n, t * COMPACT_TILE, lane, m);
+    tile_masks(flags, n, t * COMPACT_TILE, lane, m);
     uint32_t c = 0;
 #pragma unroll
     for (int u = 0; u < COMPACT_STEPS; u++) c += __popc(m[u]);
@@ -1662,7 +1680,6 @@ __global__ void __launch_bounds__(SCAN_BLOCK) k_compact_scan(uint32_t *counts, i
 // the rows where they lie, 64 flags at a step, cost 900 instructions a tile
 // whatever it held, and a store for every few rows: 100M rows, one in twenty
 // flagged, 37 us against 25.)
-template <bool VEC>
 __global__ void __launch_bounds__(BLOCK) k_compact_write(const uint8_t *__restrict__ flags, int64_t n, int64_t ntiles,
                                                          const uint32_t *__restrict__ offsets,
                                                          int32_t *__restrict__ row_ids)
@@ -1674,7 +1691,7 @@ __global__ void __launch_bounds__(BLOCK) k_compact_write(const uint8_t *__restri
     uint16_t *const list = lists[wave];
     const int64_t t0 = t * COMPACT_TILE;
     uint32_t m[COMPACT_STEPS];
-    tile_masks<VEC>(flags, n, t0, lane, m);
+    tile_masks(flags, n, t0, lane, m);
     int32_t *out = row_ids + offsets[t];
 #pragma unroll
     for (int u = 0; u < COMPACT_STEPS; u++) {
@@ -2174,9 +2191,8 @@ void launch_count_flags(const uint8_t *flags, int64_t n, uint64_t *out, bool acc
         check_launch("count_flags init");
     }
     if (n <= 0) return;
-    const int vec = aligned(flags, 16);
-    const unsigned grid = stream_grid(n, (int64_t)RED_BLOCK * (vec ? 16 * UNROLL : 1), RED_PER_CU);
-    hipLaunchKernelGGL(k_count_flags, dim3(grid), dim3(RED_BLOCK), 0, s, flags, n, out, vec);
+    const unsigned grid = stream_grid(n, (int64_t)RED_BLOCK * 16 * UNROLL, RED_PER_CU);
+    hipLaunchKernelGGL(k_count_flags, dim3(grid), dim3(RED_BLOCK), 0, s, flags, n, out);
     check_launch("count_flags");
 }
 
@@ -2219,13 +2235,9 @@ void launch_groupby_dense(const int32_t *const *keys, int k, const int32_t *mins
         const size_t used = bytes + (GB_BLOCK / 64) * GB_LIST * sizeof(uint16_t);
         const int per_cu = std::max(1, std::min(2, (int)(LDS_PER_CU / used)));
         const dim3 grid(stream_grid(n, WT_ROWS * (GB_BLOCK / 64), per_cu));
-#define SDB_GROUPBY_CASE(KV)                                                                                       \
-    if (aligned(flags, 4))                                                                                         \
-        hipLaunchKernelGGL((k_groupby_lds<KV, true>), grid, dim3(GB_BLOCK), bytes, s, g, agg, flags, n, sums, seen, \
-                           (uint32_t)prod);                                                                        \
-    else                                                                                                           \
-        hipLaunchKernelGGL((k_groupby_lds<KV, false>), grid, dim3(GB_BLOCK), bytes, s, g, agg, flags, n, sums, seen, \
-                           (uint32_t)prod);                                                                        \
+#define SDB_GROUPBY_CASE(KV)                                                                                     \
+    hipLaunchKernelGGL((k_groupby_lds<KV>), grid, dim3(GB_BLOCK), bytes, s, g, agg, flags, n, sums, seen,        \
+                       (uint32_t)prod);                                                                          \
     break;
         switch (k) {
         case 1: SDB_GROUPBY_CASE(1)
@@ -2354,14 +2366,10 @@ void launch_compact_into(const uint8_t *flags, int64_t n, int32_t *row_ids, uint
 {
     const int64_t ntiles = compact_tiles(n);
     const dim3 grid((unsigned)((ntiles + COMPACT_WAVES - 1) / COMPACT_WAVES));
-    const bool vec = aligned(flags, 16);
-    if (ntiles > 0 && vec) hipLaunchKernelGGL((k_compact_count<true>), grid, dim3(BLOCK), 0, s, flags, n, ntiles, counts);
-    else if (ntiles > 0) hipLaunchKernelGGL((k_compact_count<false>), grid, dim3(BLOCK), 0, s, flags, n, ntiles, counts);
+    if (ntiles > 0) hipLaunchKernelGGL(k_compact_count, grid, dim3(BLOCK), 0, s, flags, n, ntiles, counts);
     hipLaunchKernelGGL(k_compact_scan, dim3(1), dim3(SCAN_BLOCK), 0, s, counts, ntiles, count);
-    if (ntiles > 0 && vec)
-        hipLaunchKernelGGL((k_compact_write<true>), grid, dim3(BLOCK), 0, s, flags, n, ntiles, counts, row_ids);
-    else if (ntiles > 0)
-        hipLaunchKernelGGL((k_compact_write<false>), grid, dim3(BLOCK), 0, s, flags, n, ntiles, counts, row_ids);
+    if (ntiles > 0)
+        hipLaunchKernelGGL(k_compact_write, grid, dim3(BLOCK), 0, s, flags, n, ntiles, counts, row_ids);
     check_launch("compact");
 }
 

@@ -133,6 +133,24 @@ def test_probe_full_lds_tables(ops, length, match, flagged, wide):
     assert (tf.cpu().numpy() == want).all() and (vo.cpu().numpy() == want_v).all()
 
 
+@pytest.mark.parametrize("n", [4 << 20, (4 << 20) + 1, (4 << 20) + 2047])
+@pytest.mark.parametrize("length", [1000, 70_000])
+def test_probe_full_lds_ends(ops, n, length):
+    """Rows in whole tiles of 2,048 only, and one and 2,047 past them."""
+    import torch
+    rng = np.random.default_rng(n)
+    pairs = np.zeros(2 * length, np.int32)
+    pairs[0::2] = rng.random(length) < 0.5
+    pairs[1::2] = rng.integers(0, 1000, length)
+    probe = rng.integers(-5, length + 5, n).astype(np.int32)
+    fl = flags_of(rng, n, 0.5)
+    tf, vo = dev(fl), torch.full((n,), -77, dtype=torch.int32, device="cuda")
+    ops.full_join(dev(probe), vo, tf, n, dev(pairs), 0, length - 1)
+    want, want_v = np.zeros(n, np.uint8), np.full(n, -77, np.int32)
+    O.probe_full(probe, want_v, fl, want, pairs, 0, length - 1)
+    assert (tf.cpu().numpy() == want).all() and (vo.cpu().numpy() == want_v).all()
+
+
 @pytest.mark.parametrize("length,match", [(1_400_000, 0.04), (1_400_000, 0.7), (2_097_152, 0.01), (2_097_153, 0.01)])
 def test_probe_full_folded_filter(ops, length, match):
     """Tables of more slots than the filter has bits, up to its largest fold
