@@ -684,9 +684,14 @@ __global__ void __launch_bounds__(BLOCK) k_pairs_to_u16(const int2 *__restrict__
 //         table, up to 256 of them in flight per wave.
 // 268M rows, 1.4M slots of which 4 % match, every row flagged: 1712 -> 712 us
 // (the scattered value stores are most of the rest); 60M rows, 300,000 slots,
-// 20 %: 374 -> 212 us; 61,130 slots in LDS, 0.8 % of 268M rows flagged: 340 ->
+// 20 %: 374 -> 197 us; 61,130 slots in LDS, 0.8 % of 268M rows flagged: 340 ->
 // 237 us.  The column, flags and touched value lines alone take 600 / 180 /
-// 210 us at the rate of a copy.
+// 210 us at the rate of a copy.  Tiles go round the blocks wave by wave: with a
+// block's waves on neighbouring tiles the last round kept some CUs busy and left
+// the others idle (60M rows, 0.5 % flagged, 65,537 slots: 60 us so, 56 now; 20 %
+// flagged, 300,000 slots: 194 and 181).  A table whose values need 32 bits is
+// read in memory by half the waves of k_probe_full: 4M rows, 2,556 slots 33 us
+// against 26, 60M rows 266 against 290.
 constexpr int PROBE_BLOCK = 1024;
 constexpr int64_t PROBE_LDS_SLOTS = 65536;        // 128 KB of 16-bit values
 constexpr uint32_t PROBE_FILTER_WORDS = 1u << 15; // 128 KB of presence bits
@@ -737,7 +742,8 @@ __global__ void __launch_bounds__(PROBE_BLOCK) k_probe_full_lds(const int32_t *_
     uint32_t *const hit_of = reinterpret_cast<uint32_t *>(probe_lds) + fwords + wave * (64 + cap);
     uint32_t *const list = hit_of + 64;
     const int64_t ntiles = n / WT_ROWS, stride = (int64_t)gridDim.x * (PROBE_BLOCK / 64);
-    int64_t tile = (int64_t)blockIdx.x * (PROBE_BLOCK / 64) + wave;
+    // (a last round is shared by all blocks)
+    int64_t tile = blockIdx.x + (int64_t)gridDim.x * wave;
     uint32_t next[WT_CHUNKS];
     if (tile < ntiles) wt_flags(in, tile * WT_ROWS, lane, next);
     for (; tile < ntiles; tile += stride) {
@@ -2093,6 +2099,9 @@ void launch_build_keyvals(const int32_t *keys, const int32_t *vals, const uint8_
 // table first (16M rows, 300,000 slots: 21 us without, 26 with; 60M rows 78
 // and 66; 6M rows, 20,000 slots 13 and 11).  A larger table would leave one
 // block per CU (1.4M slots, 200M rows, 4 % flagged: 284 us without, 306 with).
+// Where hardly a row is flagged the bitmap answers rows that nobody asks for
+// (200M rows, 61,130 slots: none flagged 228 us without, 250 with; 0.5 % 238 and
+// 252; 4 % 276 and 252; all 780 and 251); how many are is not known here.
 constexpr int64_t SEMI_LDS_MIN_ROWS = 4 << 20;
 constexpr int64_t SEMI_LDS_MIN_RATIO = 128;
 constexpr int64_t SEMI_LDS_MAX_SLOTS = (int64_t)LDS_PER_CU / 2 * 8;
