@@ -61,8 +61,8 @@ static void dump_program(const FProgram &p, int64_t n, const std::string &table)
         return e && *e && *e != '0';
     }();
     if (!on) return;
-    fprintf(stderr, "[fused %s] rows=%lld vec=%d instr=%d vals=%d prefetch=%d blobs=%d lds=%u group=%d fold=%u\n",
-            table.c_str(), (long long)n, p.vec, p.ninstr, p.nvals, p.npf, p.nblobs, p.lds_bytes, p.gb.lds, p.fold);
+    fprintf(stderr, "[fused %s] rows=%lld vec=%d instr=%d vals=%d prefetch=%d blobs=%d lds=%u group=%d tries=%u fold=%u\n",
+            table.c_str(), (long long)n, p.vec, p.ninstr, p.nvals, p.npf, p.nblobs, p.lds_bytes, p.gb.lds, p.gb.hash_tries, p.fold);
     for (int i = 0; i < p.ninstr; i++) {
         const FInstr &I = p.ins[i];
         fprintf(stderr, "  %2d %-12s in=%d out=%d logic=%d va=%d vb=%d vout=%d lds=%d vkind=%d store=%d\n", i,
@@ -539,10 +539,20 @@ double expected_groups(const std::vector<Draft> &d, const FGroup &g)
     }
     return groups;
 }
-// More groups than this leave the LDS hash crowded: most rows then search it in
-// vain (32 slots) and go to the global arrays all the same.  q3.x by city over
-// 30M rows (15,000 groups): the kernel 196 us through the hash, 182 without.
-constexpr double HASH_MAX_GROUPS = 4.0 * F_HASH_CAP;
+// More groups than this leave the LDS hash crowded: most rows search it in vain
+// and go to the global arrays all the same, and the slots they did fill are
+// all written there at the end.  The hash is then there for the groups that
+// many rows share, whose atomics on one sum would wait for each other; they come
+// early and find a slot.  So a row looks at few slots, and the one that opens a
+// slot goes to the global arrays itself, which leaves nothing to write for a
+// group that meets no other row of the block.  k cities by k cities over 30M
+// rows, the kernel with 32 tries, so, and with all rows in the global arrays:
+// 10,108 groups 201, 154, 151 us; 17,500 248, 179, 176; nine rows in ten in one
+// group (17,500 expected) 275, 316 and 41,900; a third of the rows in 63 groups
+// 344, 319 and 11,000; three fifths in 1,008 904, 917 and 2,020.  (The line:
+// 4,032 groups 114, 111, 105; over 5M rows 26, 31, 29.)
+constexpr double HASH_MANY_GROUPS = 4.0 * F_HASH_CAP;
+constexpr uint32_t HASH_TRIES = 32, HASH_TRIES_SHARED = 4;
 
 // Columns the kernel prefetches.  A lazily loaded column costs the whole
 // wave a dependent memory round trip whenever any of its lanes needs it, which
@@ -873,8 +883,9 @@ bool KernelBundle::build_program(const ExecContext &ctx, FProgram &p) const
             fits = fits && exact == g.prod && g.prod <= 0x80000000ull;
             G.exact = fits;
             G.lds = !fits ? FG_GLOBAL : (g.prod <= F_DENSE_MAX ? FG_DENSE_LDS : FG_HASH_LDS);
-            if (G.lds == FG_HASH_LDS && (!hash_groupby_enabled() || expected_groups(d, G) > HASH_MAX_GROUPS))
-                G.lds = FG_GLOBAL;
+            if (G.lds == FG_HASH_LDS && !hash_groupby_enabled()) G.lds = FG_GLOBAL;
+            G.hash_shared = expected_groups(d, G) > HASH_MANY_GROUPS;
+            G.hash_tries = G.hash_shared ? HASH_TRIES_SHARED : HASH_TRIES;
             group_area = G.lds == FG_DENSE_LDS ? (uint32_t)(g.prod * 8 + (g.prod + 31) / 32 * 4 + 16)
                          : G.lds == FG_HASH_LDS ? F_HASH_CAP * 12u + 16u
                                                 : 0u;

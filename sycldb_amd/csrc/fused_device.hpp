@@ -99,11 +99,23 @@ __device__ __forceinline__ void gb_row_mode(const FGroup &g, uint8_t *lds, const
             const uint32_t mask = g.hash_cap - 1;
             uint32_t h = (s * 2654435761u) & mask;
 #pragma unroll 1
-            for (int probe = 0; probe < 32; probe++) {
+            for (uint32_t probe = 0; probe < g.hash_tries; probe++) {
                 uint32_t cur = hk[h];
                 if (cur == HASH_EMPTY) {
-                    cur = atomicCAS(&hk[h], HASH_EMPTY, s);
-                    if (cur == HASH_EMPTY) cur = s;
+                    // shared: every other lane opens slots, half as many for
+                    // rows that come alone; the rest look again after them
+                    if (!(g.hash_shared & threadIdx.x)) {
+                        cur = atomicCAS(&hk[h], HASH_EMPTY, s);
+                        if (cur == HASH_EMPTY) {
+                            if (g.hash_shared) break;
+                            cur = s;
+                        }
+                    }
+                    __builtin_amdgcn_wave_barrier();
+                    if (cur == HASH_EMPTY) {
+                        cur = *static_cast<volatile uint32_t *>(&hk[h]);
+                        if (cur == HASH_EMPTY) break;
+                    }
                 }
                 if (cur == s) {
                     atomicAdd(&hv[h], v);
@@ -111,7 +123,8 @@ __device__ __forceinline__ void gb_row_mode(const FGroup &g, uint8_t *lds, const
                 }
                 h = (h + 1) & mask;
             }
-            // table crowded: fall through to the global update
+            // table crowded, or a slot just opened or left unopened: fall
+            // through to the global update
         }
     }
     // an in-range row of exactly multiplying key ranges has its slot already;
@@ -191,8 +204,10 @@ template <int NT = BLOCK> __device__ __forceinline__ void block_epilogue(const F
         __syncthreads();
         const uint32_t *hk = reinterpret_cast<const uint32_t *>(lds + g.lds_off);
         const unsigned long long *hv = reinterpret_cast<const unsigned long long *>(hk + g.hash_cap);
+        // (a shared hash's group is in the global arrays already: a sum of 0
+        // adds nothing)
         for (uint32_t h = threadIdx.x; h < g.hash_cap; h += NT)
-            if (hk[h] != HASH_EMPTY) gb_flush_slot(g, hk[h], hv[h]);
+            if (hk[h] != HASH_EMPTY && !(g.hash_shared && hv[h] == 0)) gb_flush_slot(g, hk[h], hv[h]);
     }
 }
 

@@ -108,6 +108,9 @@ struct FGroup {
     uint64_t prod;
     uint32_t lds_off;          // byte offset of the LDS aggregation area
     uint32_t hash_cap;         // FG_HASH_LDS: slots (power of two)
+    uint32_t hash_tries;       // FG_HASH_LDS: slots a row looks at before it goes to the global arrays
+    uint32_t hash_shared;      // 1: the row that opens a slot goes to the global arrays itself, so the
+                               // hash holds only what further rows of its group add
     uint32_t exact;            // the key ranges multiply to prod (< 2^31): an in-range
                                // row's slot is its index, no remainder
 };

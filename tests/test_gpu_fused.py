@@ -40,10 +40,8 @@ def test_presence_filter_of_a_wide_probe():
                 assert fused == unfused and len(fused) > 0
 
 
-# The groups a group-by is expected to meet decide its form: 6 x 10 x 10 in
-# the LDS hash, 6 x 10 x 50 crowding it, 6 x 50 x 50 straight to the global
-# arrays; a build side with keys outside the group's range (the slot's
-# remainder) stays with the general form.
+# 6 x 10 x 10 groups, 6 x 10 x 50, 6 x 50 x 50, through the LDS hash: the last
+# are more than it holds, and a row looks at few of its slots.
 @pytest.mark.parametrize("cust,supp", [(("nation", 6), ("nation", 6)), (("nation", 6), ("region", 1)),
                                        (("region", 1), ("region", 3))])
 @pytest.mark.parametrize("codegen", ["compile", "interpret"])
@@ -92,3 +90,68 @@ def test_filtered_probe_issued_early():
     print(out.stderr[-4000:])
     assert out.returncode == 0, out.stdout
     assert "fold=3" in out.stderr  # the filtered probe comes third
+
+
+FORMS = """
+import numpy as np
+from oracle import datagen, plan_oracle as PO
+from sycldb_amd import plans as PL, schema as S
+from sycldb_amd.engine import Engine
+tables = datagen.generate_tables(S, 120_007, 45)
+rng = np.random.default_rng(1)
+for key, n in ((S.LO_CUSTKEY, 300_000), (S.LO_SUPPKEY, 20_000)):  # nine rows in ten in one group
+    tables["lineorder"][key] = np.where(rng.random(120_007) < 0.9, 77, rng.integers(1, n, 120_007)).astype(np.int32)
+where = [int(tables[t][c][76]) for t, c in (("customer", S.C_REGION), ("supplier", S.S_REGION))]
+with Engine(codegen="%s") as eng:
+    eng.load_tables(tables)
+    for group in ("nation", "city"):
+        plan = PL.build("t3", cust=("region", where[0]), supp=("region", where[1]), date=("year_range", 1992, 1997),
+                        group=group)
+        rows = eng.execute(plan).rows()
+        assert rows == PO.execute_plan(plan, tables).rows()
+        assert len(rows) > 50, len(rows)
+"""
+
+
+@pytest.mark.parametrize("codegen", ["compile", "interpret"])
+def test_groupby_of_many_groups_keeps_the_hash(codegen):
+    """Where one group takes most of the rows its sum belongs in LDS, however
+    many groups there may be: 875 (32 tries) and 17,500 (4)."""
+    out = subprocess.run([sys.executable, "-c", FORMS % codegen], cwd=ROOT, capture_output=True, text=True, timeout=110,
+                         env=dict(os.environ, SDB_DEBUG_FUSED="1"))
+    forms = [line.split("group=")[1].split(" fold")[0] for line in out.stderr.splitlines()
+             if line.startswith("[fused lineorder]")]
+    assert out.returncode == 0, out.stderr[-4000:]
+    assert forms == ["2 tries=32", "2 tries=4"]
+
+
+@pytest.mark.parametrize("spans,prod", [([(0, 599)], 600), ([(5, 3004)], 3000), ([(-7, 2), (1, 600)], 6000),
+                                        ([(-7, 2), (1, 600)], 6001), ([(3, 9), (0, 40)], 100)])
+def test_groupby_of_keys_outside_their_ranges(spans, prod):
+    """A fused group-by whose keys leave the ranges it was given, in LDS (dense,
+    hashed with many and with few tries) and where the ranges do not multiply
+    to the slots: those rows take their slot's remainder, the others theirs."""
+    import numpy as np
+    import torch
+    from oracle import oracle as O
+    from sycldb_amd import _lib as L, ops
+    from sycldb_amd.engine import codegen_wait
+    n, rng = 70_003, np.random.default_rng(prod)
+    keys = [rng.integers(a - 3, b + 4, n).astype(np.int32) for a, b in spans]
+    agg = rng.integers(-2**31, 2**31, n).astype(np.int32)
+    fl = (rng.random(n) < 0.7).astype(np.uint8)
+    mins, maxs = [a for a, _ in spans], [b for _, b in spans]
+    ws, wn = np.zeros(prod, np.uint64), np.zeros(prod, np.uint32)
+    O.groupby_dense(keys, mins, maxs, agg, fl, [np.zeros(prod, np.int32) for _ in spans], ws, wn, prod)
+    dk, da, df = [torch.from_numpy(k).cuda() for k in keys], torch.from_numpy(agg).cuda(), torch.from_numpy(fl).cuda()
+    outk = [torch.zeros(prod, dtype=torch.int32, device="cuda") for _ in spans]
+    sums, seen = (torch.zeros(prod, dtype=d, device="cuda") for d in (torch.int64, torch.int32))
+    op = L.Op(kind=L.OP_GROUPBY, nkeys=len(spans), col=da.data_ptr(), in_flags=df.data_ptr(), sums=sums.data_ptr(),
+              seen=seen.data_ptr(), prod=prod)
+    for j in range(len(spans)):
+        op.keys[j], op.out_keys[j], op.mins[j], op.maxs[j] = dk[j].data_ptr(), outk[j].data_ptr(), mins[j], maxs[j]
+    for rep in range(2):  # the interpreter, then the compiled kernel
+        sums.zero_(), seen.zero_()
+        ops.bundle_exec([op], n)
+        assert (sums.cpu().numpy().view(np.uint64) == ws).all() and (seen.cpu().numpy().view(np.uint32) == wn).all()
+        assert codegen_wait(100)
