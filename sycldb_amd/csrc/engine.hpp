@@ -335,10 +335,13 @@ struct Engine {
     int64_t launches = 0;
     double last_device_ms = 0, last_wall_ms = 0;
     hipEvent_t ev_start = nullptr, ev_stop = nullptr;
-    // pinned host staging of result downloads (grown on demand, freed with
+    // pinned host staging of result downloads (grown on demand, given back
+    // when it has long been far larger than what is asked for, freed with
     // the engine): one asynchronous copy per array and one sync
     void *pinned = nullptr;
     size_t pinned_bytes = 0;
+    size_t pinned_most = 0; // largest request of the last pinned_calls
+    int pinned_calls = 0;
     void *pinned_buffer(size_t bytes);
     // Waits until the stream's work so far is done, polling an event: the
     // engine waits only between device phases that follow each other

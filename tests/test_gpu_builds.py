@@ -175,3 +175,19 @@ def test_batches_over_a_table_loaded_again():
             got, batched = eng.execute_batch(plans)
             assert batched == len(plans)
             assert [g.rows() for g in got] == [PO.execute_plan(p, tables).rows() for p in plans]
+
+
+def test_result_staging_goes_back():
+    """A batch of large results, hundreds of small ones, the batch again."""
+    from sycldb_amd.engine import Engine
+    tables = datagen.generate_tables(S, 60_003, 45)
+    large = [PL.build("t3", cust=("region", i), supp=("region", i), date=("year_range", 1992, 1997), group="city")
+             for i in range(5)]
+    small = PL.build("t1")
+    w_large, w_small = [PO.execute_plan(p, tables).rows() for p in large], PO.execute_plan(small, tables).rows()
+    with Engine() as eng:
+        eng.load_tables(tables)
+        assert [r.rows() for r in eng.execute_batch(large)[0]] == w_large
+        for _ in range(600):  # (its buffer then is a small one)
+            assert eng.execute(small).rows() == w_small
+        assert [r.rows() for r in eng.execute_batch(large)[0]] == w_large
