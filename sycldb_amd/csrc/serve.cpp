@@ -92,11 +92,13 @@ uint64_t estimate_footprint(Engine &eng, const PlanResult &plan)
 // Batch cost model of the serving loop: the marginal cost of one more
 // program in a shared scan, as a fraction of its plain run (measured at 600M
 // rows: 0.4-0.9 ms per extra program against 1.6-2.7 ms alone), and the
-// fixed part assumed before any batch has run on an engine, in plain runs
-// (with that marginal cost, batches of 8: 2.1 over 200,000 rows; over 600M
-// rows 1.8 for q1.x and q4.x, 2.4 for q3.x, 5 for q2.x).
+// fixed part assumed before any batch has run on an engine, in plain runs.
+// Batches of 2, 4 and 8 of all templates, with that marginal cost: over 200,000
+// rows 1.8, 2.7, 2.4; 6M 1.7, 2.3, 2.8; 60M 2.7, 3.2, 3.6; 600M 3.3, 4.0, 4.2
+// (of one template 1.3 to 2.8, but q2.x over 600M 3.7 to 4.4): between the small
+// tables' and the large ones', nearer the small, whose queues are the long ones.
 constexpr double BATCH_MARGINAL = 0.3;
-constexpr double BATCH_FIXED_INITIAL = 2.0;
+constexpr double BATCH_FIXED_INITIAL = 2.5;
 // Wave slots per CU (of 32) a batched scan may take while other engines'
 // workers run: a batched kernel that fills every slot makes the others'
 // kernels wait for its whole scan.
