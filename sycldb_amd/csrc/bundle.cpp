@@ -53,14 +53,20 @@ static const char *fkind_name(uint8_t k)
     return k < sizeof(names) / sizeof(names[0]) ? names[k] : "?";
 }
 
-// SDB_DEBUG_FUSED=1 prints each fused program to stderr.
-static void dump_program(const FProgram &p, int64_t n, const std::string &table)
+// SDB_DEBUG_FUSED=1 prints each fused program, and the flag buffers of each
+// bundle that runs one kernel per operator, to stderr.
+static bool debug_fused()
 {
     static const bool on = [] {
         const char *e = getenv("SDB_DEBUG_FUSED");
         return e && *e && *e != '0';
     }();
-    if (!on) return;
+    return on;
+}
+
+static void dump_program(const FProgram &p, int64_t n, const std::string &table)
+{
+    if (!debug_fused()) return;
     fprintf(stderr, "[fused %s] rows=%lld vec=%d instr=%d vals=%d prefetch=%d blobs=%d lds=%u group=%d tries=%u fold=%u\n",
             table.c_str(), (long long)n, p.vec, p.ninstr, p.nvals, p.npf, p.nblobs, p.lds_bytes, p.gb.lds, p.gb.hash_tries, p.fold);
     for (int i = 0; i < p.ninstr; i++) {
@@ -217,6 +223,9 @@ void KernelBundle::execute_unfused(const ExecContext &ctx) const
         ctx.virgin_filled = true;
     }
     const auto shared = shared_flags(kernels_, ctx);
+    if (debug_fused())
+        fprintf(stderr, "[unfused %s] operators=%zu one_flag_buffer=%d\n", ctx.table ? ctx.table->c_str() : "?",
+                kernels_.size(), shared.first != nullptr);
     for (const KernelData &k0 : kernels_) {
         if (k0.type == KernelType::EmptyKernel) continue;
         KernelData k = k0;

@@ -191,3 +191,68 @@ def test_result_staging_goes_back():
         for _ in range(600):  # (its buffer then is a small one)
             assert eng.execute(small).rows() == w_small
         assert [r.rows() for r in eng.execute_batch(large)[0]] == w_large
+
+
+# 1,000-row segments: those builds keep kernels of their own, in order
+@pytest.mark.parametrize("customer,supplier,part,ddate", [(999, 1001, 2000, 2556), (3001, 1, 1000, 366)])
+def test_segmented_build_sides(customer, supplier, part, ddate):
+    from sycldb_amd.engine import Engine
+    sizes = {"customer": customer, "supplier": supplier, "part": part, "ddate": ddate}
+    rows, seed = 7_001, 45
+    tables = datagen.generate_tables(S, rows, seed, sizes)
+    with Engine(segment_size=1000) as eng:
+        eng.generate(rows, seed, sizes=sizes)
+        for t, p in PLANS:
+            plan = PL.build(t, **p)
+            assert eng.execute(plan).rows() == PO.execute_plan(plan, tables).rows(), plan
+
+
+@pytest.mark.parametrize("rows", [(4 << 20) - 1, 4 << 20, (4 << 20) + 1])
+def test_largest_build_side_of_a_shared_launch(rows):
+    """Build sides of fewer than 4M rows share a launch, larger ones have
+    kernels of their own: the results of one kernel per operator."""
+    from sycldb_amd.engine import Engine
+    plans = [PL.build(t, **p) for t, p in PLANS if t in ("t2", "t3", "t4")]
+    with Engine() as eng:
+        eng.generate(300_001, 45, sizes={"customer": rows, "part": rows})
+        eng.set_fusion(False)
+        want = [eng.execute(p).rows() for p in plans]
+        eng.set_fusion(True)
+        for _ in range(2):
+            assert [eng.execute(p).rows() for p in plans] == want
+        assert any(want)
+
+
+ONE_BUFFER = """
+import sys
+sys.path.insert(0, "tests")
+import quirk_plans as Q
+from oracle import datagen, plan_oracle as PO
+from sycldb_amd import plans as PL, schema as S
+from sycldb_amd.engine import Engine
+tables = datagen.generate_tables(S, 50_007, 45)
+b = PL.PlanBuilder()  # its flags are the result
+b.scan("lineorder")
+b.filter(PL.expr("AND", PL.expr("=", PL.col(S.LO_DISCOUNT), PL.lit(2)), PL.expr("<", PL.col(S.LO_QUANTITY), PL.lit(9))))
+plans = [PL.build("t4"), PL.build("t1"), Q.left_fold_or_and(), Q.left_fold_and_or(), Q.filter_after_join(), b.plan()]
+with Engine(fusion=False) as eng:
+    eng.load_tables(tables)
+    for p in plans:
+        print("plan", file=sys.stderr)
+        assert eng.execute(p).rows() == PO.execute_plan(p, tables).rows()
+"""
+
+
+def test_which_operators_share_a_flag_buffer():
+    """One kernel per operator: a chain whose flags nobody reads after it keeps
+    them in one buffer, a filter that is the plan's result does not."""
+    import os
+    import subprocess
+    import sys
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    out = subprocess.run([sys.executable, "-c", ONE_BUFFER], cwd=root, capture_output=True, text=True, timeout=110,
+                         env=dict(os.environ, SDB_DEBUG_FUSED="1"))
+    assert out.returncode == 0, out.stderr[-4000:]
+    forms = [[l.split("one_flag_buffer=")[1] for l in part.splitlines() if l.startswith("[unfused lineorder]")]
+             for part in out.stderr.split("plan\n")[1:]]
+    assert forms == [["1"]] * 5 + [["0"]]

@@ -155,3 +155,27 @@ def test_groupby_of_keys_outside_their_ranges(spans, prod):
         ops.bundle_exec([op], n)
         assert (sums.cpu().numpy().view(np.uint64) == ws).all() and (seen.cpu().numpy().view(np.uint32) == wn).all()
         assert codegen_wait(100)
+
+
+FILTERED = """
+from sycldb_amd import plans as PL, schema as S
+from sycldb_amd.engine import Engine
+T2 = (S.LO_PARTKEY, S.LO_SUPPKEY, S.LO_ORDERDATE, S.LO_REVENUE)
+for rows, parts in (((1 << 25) + 3, 1_400_000), ((1 << 25) + 3, (1 << 20) - 1), ((1 << 25) - 1, 1_400_000)):
+    with Engine(codegen="interpret") as eng:
+        eng.generate(rows, 11, sizes={"part": parts}, fact_columns=T2)
+        for cg in ("compile", "interpret"):
+            eng.set_codegen(cg)
+            for part in (("category", 3), ("mfgr2", 0, 1)):
+                eng.execute(PL.t2_plan(part, 2))
+"""
+
+
+def test_presence_filter_is_taken():
+    """Of the plans above, those with a presence filter: enough rows, a wide
+    table, few matches, a compiled kernel."""
+    out = subprocess.run([sys.executable, "-c", FILTERED], cwd=ROOT, capture_output=True, text=True, timeout=110,
+                         env=dict(os.environ, SDB_DEBUG_FUSED="1"))
+    assert out.returncode == 0, out.stderr[-4000:]
+    folds = [line.split("fold=")[1] != "0" for line in out.stderr.splitlines() if line.startswith("[fused lineorder]")]
+    assert folds == [True, False, False, False] + [False] * 8
