@@ -451,11 +451,15 @@ def main():
     log("fused: %.3f ms/step, %.3e rows/s, %d groups; profile %s" % (ms_per_step, value, groups, prof))
 
     launches, krows, kms = prof.get("fused:lineorder", (0, 0, 0.0))
+    # the rate of the bytes the kernel moves, where their counters are
+    # committed for this workload; else of its columns' bytes, each read whole
+    # (a kernel that reads columns lazily moves fewer)
     bytes_per_row = 4 * len(fact_cols)
-    achieved = (bytes_per_row * krows / (kms / 1000.0)) / 1e9 if kms > 0 else None
+    dense = (bytes_per_row * krows / (kms / 1000.0)) / 1e9 if kms > 0 else None
     traffic = measured_traffic(args.workload, rows)
+    achieved = traffic["bytes_per_launch"] * launches / (kms / 1000.0) / 1e9 if traffic and kms > 0 else dense
     roofline = {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
-                "frac": (achieved / HBM_PEAK_GBS) if achieved else None,
+                "frac": (achieved / HBM_PEAK_GBS) if achieved else None, "dense_scan_GBps": dense,
                 "traffic": traffic["bytes_per_launch"] if traffic else None,
                 "traffic_source": traffic["source"] if traffic else None,
                 "kernel": "sdb_fused_program (fused lineorder bundle, compiled for its program shape)" if args.codegen != "interpret" else "k_fused (fused lineorder bundle, interpreted)", "launches_per_step": launches // max(args.steps, 1),
