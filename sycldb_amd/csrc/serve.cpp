@@ -97,6 +97,10 @@ uint64_t estimate_footprint(Engine &eng, const PlanResult &plan)
 // rows 1.8, 2.7, 2.4; 6M 1.7, 2.3, 2.8; 60M 2.7, 3.2, 3.6; 600M 3.3, 4.0, 4.2
 // (of one template 1.3 to 2.8, but q2.x over 600M 3.7 to 4.4): between the small
 // tables' and the large ones', nearer the small, whose queues are the long ones.
+// Mean latency of 2,000 requests at 3,000/s over three tables, three runs each:
+// 1.0 19.8 to 23.6 ms with a worker per engine and 18.2 to 22.3 with one; 2.0 19.7
+// to 31.6 and 18.0 to 18.3; 2.5 19.3 to 21.4 and 17.8 to 22.7; 4.0 19.2 to 20.8 and
+// 18.1 to 18.4 (but then a burst of small requests may drain unbatched).
 constexpr double BATCH_MARGINAL = 0.3;
 constexpr double BATCH_FIXED_INITIAL = 2.5;
 // Wave slots per CU (of 32) a batched scan may take while other engines'
