@@ -2535,7 +2535,8 @@ constexpr uint64_t BATCH_STAGE_LDS_MAX = 144 * 1024;
 constexpr int N_BATCH_CAND = (int)(sizeof(BATCH_CANDIDATES) / sizeof(BATCH_CANDIDATES[0]));
 
 std::mutex g_lib_mu;
-std::map<std::string, BatchLibrary> g_libs;
+// (never destroyed: a program's last engine may go after this library's statics)
+std::map<std::string, BatchLibrary> &g_libs = *new std::map<std::string, BatchLibrary>;
 
 // Rewrites a program's prefetch registers to library slots (adding its
 // columns); a column beyond BATCH_MAX_PF slots is read from memory instead.
