@@ -178,7 +178,7 @@ def test_batches_over_a_table_loaded_again():
 
 
 def test_result_staging_goes_back():
-    """A batch of large results, hundreds of small ones, the batch again."""
+    """A batch of large results, thousands of small ones, the batch again."""
     from sycldb_amd.engine import Engine
     tables = datagen.generate_tables(S, 60_003, 45)
     large = [PL.build("t3", cust=("region", i), supp=("region", i), date=("year_range", 1992, 1997), group="city")
@@ -188,7 +188,9 @@ def test_result_staging_goes_back():
     with Engine() as eng:
         eng.load_tables(tables)
         assert [r.rows() for r in eng.execute_batch(large)[0]] == w_large
-        for _ in range(600):  # (its buffer then is a small one)
+        for _ in range(2 * 4096 + 8):  # (its buffer then is a small one)
+            eng.execute(small)
+        for _ in range(3):
             assert eng.execute(small).rows() == w_small
         assert [r.rows() for r in eng.execute_batch(large)[0]] == w_large
 
